@@ -92,16 +92,14 @@ __host__ __device__ constexpr int rys_block_doubles(int n) {
   return (int)rys_largex(n) * 2 * n * kRysNc;
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs of an MI355X; remap
-// so that XCD x runs a contiguous range of block indices (tuples that are
-// adjacent in a bin share bra pairs, whose primitive data then stays in that
-// XCD's L2).  A bijection on [0, gridDim.x).
-__device__ __forceinline__ int xcd_block() {
-  const int nb = gridDim.x, b = blockIdx.x;
-  const int x = b & 7, local = b >> 3;
-  const int q = nb >> 3, r = nb & 7;
-  return x * q + (x < r ? x : r) + local;
-}
+// Workgroups are dispatched in index order, round-robin over the 8 XCDs, and
+// a bin's tuples are sorted by ascending primitive work: taking the blocks
+// from the end starts the longest ones first and spreads them evenly over the
+// XCDs.  (A contiguous range of blocks per XCD, for the sake of its L2, gave
+// one XCD all of the longest tuples: (d p|p s), 946,107 tuples of a 64-atom
+// molecule, took 10.1 ms that way and takes 2.7 ms so, 25.6 TFLOP/s; the
+// primitive records are a few MB and stay in every L2.)
+__device__ __forceinline__ int heavy_first_block() { return gridDim.x - 1 - blockIdx.x; }
 
 // Per-tuple scalars of one primitive tuple.
 struct PrimTuple {
@@ -480,7 +478,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
 
   const int slot = threadIdx.x / T;
   const int t = threadIdx.x - slot * T;
-  const int64_t q = (int64_t)xcd_block() * Q + slot;
+  const int64_t q = (int64_t)heavy_first_block() * Q + slot;
   const bool active = q < a.nq;
   const int2 pq = a.quartets[active ? q : 0];
   const int boff = a.pair_off[pq.x];
