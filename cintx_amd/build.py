@@ -125,7 +125,7 @@ def _p2(v):
     return p
 
 
-def register_chunks(deriv, prec, ls):
+def register_chunks(deriv, prec, ls, limit=None):
     """Row chunks for the one-lane path on a class too large for one pass:
     the g tensor of one root (3*G4 values) and a chunk's FP64 accumulators
     should fit about 130 doubles of registers (VGPRs plus AGPRs at one wave
@@ -143,11 +143,27 @@ def register_chunks(deriv, prec, ls):
         return None
     # FP32 keeps a per-primitive-tuple partial sum beside each FP64 accumulator
     per_acc = 1.0 if prec == 0 else 1.5
+    # nabla_i holds its factors as well: from 108 doubles on it spilled 0.4 to
+    # 1.2 KB per lane and ran 20 to 50 times slower
+    limit = limit or (105 if deriv else 130)
     for nch in (2, 3):
         rpc = -(-nrow // nch)
-        if gdoubles + per_acc * rpc * nb * (3 if deriv else 1) <= 130:
+        if gdoubles + per_acc * rpc * nb * (3 if deriv else 1) <= limit:
             return nch
     return None
+
+
+def by_work(deriv, prec, ls):
+    """Whether a plan places a class's blocks by surviving primitive tuples (by
+    primitive counts otherwise).  The order of the blocks in a plan's buffer
+    stays what it is whichever launch shapes a class has."""
+    if prec == 2:
+        return by_work(deriv, 0, ls)
+    nc = [(l + 1) * (l + 2) // 2 for l in ls]
+    ne = nc[0] * nc[1] * nc[2] * nc[3] * (3 if deriv else 1)
+    if is_high_l(deriv, ls):
+        return ne <= 81 and not needs_pb(ls) and (deriv == 1 or nc[0] * nc[1] <= 36)
+    return ne <= 81 or register_chunks(deriv, prec, ls, limit=130) is not None
 
 
 def variants(deriv, prec, ls):
@@ -268,6 +284,8 @@ def generate(nparts=24, nchunkparts=12):
     reg += [f"void register_part_{p}(Registry& reg);" for p in range(nparts)]
     reg += ["void register_class_kernels(Registry& reg) {"]
     reg += [f"  register_part_{p}(reg);" for p in range(nparts)]
+    reg += ["  reg.by_work[{}][{}][{}][{}][{}][{}] = true;".format(deriv, prec, *ls)
+            for deriv, prec, ls in classes if by_work(deriv, prec, ls)]
     reg += ["}", "}  // namespace cx", ""]
     path = os.path.join(GEN, "inst_registry.cpp")
     text = "\n".join(reg)

@@ -39,6 +39,19 @@ struct RysTable {
   int off[kMaxRoots + 1];  // start of n's block in coef
 };
 
+// Lanes per tuple of a one-lane launch: the tuples of a bin are sorted by
+// ascending surviving primitive tuples and cut into up to kSplits ranges;
+// range k ends at tuple end[k] and gives each tuple 2^k adjacent lanes of a
+// wavefront, which share the tuple's primitive tuples.
+constexpr int kSplits = 7;
+struct LaneSplit {
+  int end[kSplits];
+};
+constexpr int kOneLaneBlock = 256;  // lanes of a one-lane kernel's workgroup
+__host__ __device__ constexpr int split_blocks(int n, int lg) {
+  return (int)((((int64_t)n << lg) + kOneLaneBlock - 1) / kOneLaneBlock);
+}
+
 // Per-launch arguments of a class kernel.
 struct EriArgs {
   // per primitive pair one 64-byte record (a lane reads one cache line per
@@ -57,6 +70,7 @@ struct EriArgs {
   int64_t out_base;        // element offset of this launch's first block
   int64_t block;           // elements per block (components included)
   int64_t nq;
+  LaneSplit split;         // one-lane kernels
   double common;           // pi^3 2/sqrt(pi) prod common_fac_sp
   double expcutoff;
   int lij_ceil, lkl_ceil;  // li_ceil+lj_ceil, lk_ceil+ll_ceil for the screen

@@ -101,6 +101,40 @@ __host__ __device__ constexpr int rys_block_doubles(int n) {
 // primitive records are a few MB and stay in every L2.)
 __device__ __forceinline__ int heavy_first_block() { return gridDim.x - 1 - blockIdx.x; }
 
+// The range of a one-lane launch that a workgroup serves: its first tuple,
+// the end of the range and the binary logarithm of the lanes per tuple.  The
+// last ranges hold the longest tuples and come first.
+struct SplitBlock {
+  int first, end, lg;
+};
+__device__ __forceinline__ SplitBlock split_block(const LaneSplit& sp) {
+  int b = blockIdx.x, k = kSplits - 1;
+  int nblk = 0;
+  for (; k >= 0; --k) {
+    const int begin = k > 0 ? sp.end[k - 1] : 0;
+    nblk = split_blocks(sp.end[k] - begin, k);
+    if (b < nblk || k == 0) break;
+    b -= nblk;
+  }
+  SplitBlock r;
+  r.lg = k;
+  r.end = sp.end[k];
+  r.first = (k > 0 ? sp.end[k - 1] : 0) + ((nblk - 1 - b) * kOneLaneBlock >> k);
+  return r;
+}
+
+// v summed over the 2^lg adjacent lanes that share a tuple (every lane gets
+// the sum).  One loop body for all distances: with a body for each (DPP moves
+// instead of the shuffles) the chunked kernels spilled 1 KB per lane.
+template <int N>
+__device__ __forceinline__ void split_sum(double* v, int lg) {
+#pragma unroll 1
+  for (int d = 1; d < 1 << lg; d <<= 1) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += __shfl_xor(v[i], d);
+  }
+}
+
 // Per-tuple scalars of one primitive tuple.
 struct PrimTuple {
   double aij, akl, a0, a1;
@@ -476,10 +510,14 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
 #pragma unroll
   for (int kk = 0; kk < ACC; ++kk) acc[kk] = 0.0;
 
-  const int slot = threadIdx.x / T;
-  const int t = threadIdx.x - slot * T;
-  const int64_t q = (int64_t)heavy_first_block() * Q + slot;
-  const bool active = q < a.nq;
+  // one-lane kernels: 2^lg adjacent lanes share a tuple, of which this is
+  // lane t; the others: T lanes per tuple
+  SplitBlock sb{0, 0, 0};
+  if constexpr (REG) sb = split_block(a.split);
+  const int slot = REG ? (int)threadIdx.x >> sb.lg : (int)threadIdx.x / T;
+  const int t = REG ? (int)threadIdx.x & ((1 << sb.lg) - 1) : (int)threadIdx.x - slot * T;
+  const int64_t q = REG ? (int64_t)sb.first + slot : (int64_t)heavy_first_block() * Q + slot;
+  const bool active = q < (REG ? (int64_t)sb.end : a.nq);
   const int2 pq = a.quartets[active ? q : 0];
   const int boff = a.pair_off[pq.x];
   const int koff = a.pair_off[pq.y];
@@ -559,20 +597,36 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   // Each lane walks only its own surviving primitive tuples.  The primitive
   // pairs of every pair are stored in ascending cce, so the bra primitives
   // that pass the screen against ket primitive kp are a prefix of the bra
-  // list, and a ket primitive whose first bra primitive fails ends the
-  // tuple (later ket primitives have larger cce).  A wavefront then runs
-  // as many iterations as its lane with the most survivors (tuples are
-  // sorted by survivor count), not the product of the primitive counts.
-  // The bra record of the next candidate is loaded one iteration ahead (its
-  // latency then hides behind the current primitive tuple's work).
+  // list, and a ket primitive against which the first bra primitive fails
+  // ends the tuple (later ket primitives have larger cce).  Of the NS lanes
+  // that share a tuple, lane t takes every NS-th bra primitive, starting at
+  // a place that turns with kp (by about 5/8 of NS, odd), so that short
+  // prefixes fall on different lanes: on the primitive lists of a 48-atom
+  // molecule the longest of 16 lanes has 1.11 times the average, against
+  // 1.93 times without the turn and 1.07 times for an exact deal.  A
+  // wavefront runs as many iterations as its lane with the most survivors
+  // (tuples are sorted by survivor count), not the product of the primitive
+  // counts.  The bra record of the next candidate is loaded one iteration
+  // ahead (its latency then hides behind the current primitive tuple's work).
   (void)mij;
   (void)mkl;
+  const int NS = 1 << sb.lg, turn = (NS * 5 / 8) | 1;
   int kp = 0, ip = 0;
   double akl = 0, wk = 0, wl = 0, kkl = 0, hkl = 0, eijcut = 0;
   double qk[3] = {0, 0, 0}, qb[3] = {0, 0, 0};  // Q - R_k, Q - R(ket base)
-  bool klok = false;
-  auto set_ket = [&](int k) {
-    const double* pk = a.prim + 8 * (size_t)(koff + k);
+  double nb[8];  // record of bra candidate ip (prefetched)
+  auto load_bra = [&](int i) {
+    const double* q = a.prim + 8 * (size_t)(boff + i);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) nb[d] = q[d];
+  };
+  // the key of the first bra primitive, past the screen where there is none
+  // (libcint zeroes the prefactor of a bra pair with cce >= expcutoff,
+  // optimizer.c:317-341, so it contributes nothing)
+  const double cce0 = np_ij > 0 ? a.prim[8 * (size_t)boff + 6] - a.lij_ceil * logd_ij : a.expcutoff;
+  auto set_ket = [&]() {  // ket primitive kp and this lane's first bra candidate
+    if (kp >= np_kl) return;
+    const double* pk = a.prim + 8 * (size_t)(koff + kp);
     akl = pk[0];
     wk = pk[1];
     wl = pk[2];
@@ -584,47 +638,34 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
     kkl = pk[4];
     hkl = pk[5];
     const double ccekl = a.three_center ? 0.0 : pk[6] - a.lkl_ceil * logd_kl;
-    klok = ccekl <= a.expcutoff;
     eijcut = a.expcutoff - ccekl;
+    if (!(ccekl <= a.expcutoff && cce0 <= eijcut && cce0 < a.expcutoff)) {
+      kp = np_kl;  // nothing survives from this ket primitive on
+      return;
+    }
+    ip = (t + kp * turn) & (NS - 1);
+    if (ip < np_ij) load_bra(ip);
   };
-  double nb[8];  // record of bra candidate ip (prefetched)
-  auto load_bra = [&](int i) {
-    const double* q = a.prim + 8 * (size_t)(boff + i);
-#pragma unroll
-    for (int d = 0; d < 8; ++d) nb[d] = q[d];
-  };
-  if (active && np_kl > 0) {
-    set_ket(0);
-    load_bra(0);
-  }
+  if (!active) kp = np_kl;
+  set_ket();
   for (;;) {
     bool have = false;
-    while (active && kp < np_kl) {
-      if (klok && ip < np_ij) {
+    while (kp < np_kl) {
+      if (ip < np_ij) {
         const double cceij = nb[6] - a.lij_ceil * logd_ij;
-        // (libcint zeroes the prefactor of a bra pair with cce >= expcutoff,
-        // optimizer.c:317-341, so it contributes nothing)
         if (cceij <= eijcut && cceij < a.expcutoff) {
           have = true;
           break;
         }
       }
-      if (ip == 0) {  // nothing survives from this ket primitive on
-        kp = np_kl;
-        break;
-      }
       ++kp;
-      ip = 0;
-      if (kp < np_kl) {
-        set_ket(kp);
-        load_bra(0);
-      }
+      set_ket();
     }
     if (!have) break;
     double pi[8];
 #pragma unroll
     for (int d = 0; d < 8; ++d) pi[d] = nb[d];
-    ++ip;
+    ip += NS;
     if (ip < np_ij) load_bra(ip);
     {
       PrimTuple p;
@@ -720,6 +761,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
       }
     }
   }
+  split_sum<ACC>(acc, sb.lg);
   // cart -> sph of the chunk, in registers: the row's own axes (i, j; i only
   // for nabla_i rows) per row, then the row axes as a weighted sum over the
   // chunk's rows, added to what earlier chunks wrote (or, for a fused J/K,
@@ -835,20 +877,26 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
               }
             }
             __syncthreads();
-            if constexpr (ONE_SITE)  // rows [0, ONE_NR), a compile-time range
-              jk_digest_rows_fixed<NSI, NSJ, NSK, NSL, ONE_NR>(
-                  lane, 256, active, sh[0], sh[1], sh[2], sh[3], off[0], off[1], off[2], off[3],
-                  a.jk_D, a.jk_J, a.jk_K, a.nao);
-            else
-              jk_digest_rows_call<NSI, NSJ, NSK, NSL>(lane, 256, r0, nr, active, sh[0], sh[1],
-                                                      sh[2], sh[3], off[0], off[1], off[2], off[3],
-                                                      a.jk_D, a.jk_J, a.jk_K, a.nao);
+            if constexpr (ONE_SITE) {  // rows [0, ONE_NR), a compile-time range
+              if (sb.lg == 0)
+                jk_digest_rows_fixed<NSI, NSJ, NSK, NSL, ONE_NR>(
+                    lane, 256, active, sh[0], sh[1], sh[2], sh[3], off[0], off[1], off[2], off[3],
+                    a.jk_D, a.jk_J, a.jk_K, a.nao);
+              else
+                jk_digest_rows<NSI, NSJ, NSK, NSL>(lane, 256, r0, nr, t, sb.lg, active, sh[0],
+                                                   sh[1], sh[2], sh[3], off[0], off[1], off[2],
+                                                   off[3], a.jk_D, a.jk_J, a.jk_K, a.nao);
+            } else {
+              jk_digest_rows_call<NSI, NSJ, NSK, NSL>(lane, 256, r0, nr, t, sb.lg, active, sh[0],
+                                                      sh[1], sh[2], sh[3], off[0], off[1], off[2],
+                                                      off[3], a.jk_D, a.jk_J, a.jk_K, a.nao);
+            }
             __syncthreads();
           }
           continue;
         }
       }
-      if (!active) continue;
+      if (!active || t != 0) continue;
       double* o = a.out + a.out_base + q * a.block + comp * a.st_comp;
 #pragma unroll
       for (int ml = 0; ml < NSL; ++ml)
@@ -1122,6 +1170,8 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
       if (nsurv) atomicAdd(&scnt[slot], nsurv);
       tuple_sync<T>();
       tot = scnt[slot];
+    } else {
+      for (int d = 1; d < 1 << sb.lg; d <<= 1) tot += __shfl_xor(tot, d);
     }
     if (t == 0 && tot) {
       atomicAdd(a.counters, (unsigned long long)tot);
@@ -1209,7 +1259,13 @@ template <int LI, int LJ, int LK, int LL, int DERIV, typename R, int TT, int PP>
 hipError_t launch_class(const EriArgs& a, hipStream_t s) {
   using S = ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>;
   constexpr int Q = S::template Q<R>();
-  const int64_t nblk = (a.nq + Q - 1) / Q;
+  int64_t nblk = (a.nq + Q - 1) / Q;
+  if constexpr (S::T == 1) {
+    static_assert(Q == kOneLaneBlock, "one-lane workgroup");
+    nblk = 0;
+    for (int k = 0; k < kSplits; ++k)
+      nblk += split_blocks(a.split.end[k] - (k > 0 ? a.split.end[k - 1] : 0), k);
+  }
   // the one-lane kernels stage their blocks for a fused J/K in dynamic LDS
   size_t dyn = 0;
   if constexpr (S::T == 1 && S::JK) {

@@ -129,6 +129,8 @@ __device__ __forceinline__ void jk_put(bool live, double* __restrict__ out, size
 // the NI NJ (i, j) values of pair r0 + r at stage[base + (r NI NJ + i + NI j)
 // ls] (ls: lane stride).  One lane per quartet; every lane of the wavefront
 // calls (`live` false for a lane without a quartet), r0 and nr are uniform.
+// Where 2^lg adjacent lanes hold the same quartet (each with a copy of the
+// rows), lane t of them takes every 2^lg-th row.
 // Row by row: the 2 NI + 2 NJ + 1 density values a row needs are loaded
 // together (independent loads, one latency per row); A[I,J] is summed over
 // the rows in registers.  Lanes whose quartets share an output block (the
@@ -143,11 +145,12 @@ __device__ __forceinline__ void jk_put(bool live, double* __restrict__ out, size
 // need together); one with several (row chunks, passes) calls the
 // out-of-line copy below, so its code is not replicated per site.
 template <int NI, int NJ, int NK, int NL>
-__device__ __forceinline__ void jk_digest_rows(int base, int ls, int r0, int nr, bool live, int s0,
-                                            int s1, int s2, int s3, int o0, int o1, int o2,
-                                            int o3, const double* __restrict__ D,
-                                            double* __restrict__ J, double* __restrict__ K,
-                                            int nao) {
+__device__ __forceinline__ void jk_digest_rows(int base, int ls, int r0, int nr, int t, int lg,
+                                               bool live, int s0, int s1, int s2, int s3, int o0,
+                                               int o1, int o2, int o3,
+                                               const double* __restrict__ D,
+                                               double* __restrict__ J,
+                                               double* __restrict__ K, int nao) {
   extern __shared__ double jk_stage[];
   constexpr int NB = NI * NJ;
   const double w = jk_weight(s0, s1, s2, s3);
@@ -157,11 +160,15 @@ __device__ __forceinline__ void jk_digest_rows(int base, int ls, int r0, int nr,
   // quartet gets a key no index takes, unique per lane)
   const unsigned long long dead = ~0ull - __lane_id();
   const WaveRun rIJ = wave_run(live ? oI * n + oJ : dead);
-  const WaveRun rKL = wave_run(live ? oK * n + oL : dead);
-  const WaveRun rIK = wave_run(live ? oI * n + oK : dead);
-  const WaveRun rIL = wave_run(live ? oI * n + oL : dead);
-  const WaveRun rJK = wave_run(live ? oJ * n + oK : dead);
-  const WaveRun rJL = wave_run(live ? oJ * n + oL : dead);
+  WaveRun rKL = wave_run(live ? oK * n + oL : dead);
+  WaveRun rIK = wave_run(live ? oI * n + oK : dead);
+  WaveRun rIL = wave_run(live ? oI * n + oL : dead);
+  WaveRun rJK = wave_run(live ? oJ * n + oK : dead);
+  WaveRun rJL = wave_run(live ? oJ * n + oL : dead);
+  if (lg > 0) {  // adjacent lanes hold different rows: elements of their own
+    rKL.tail = rIK.tail = rIL.tail = rJK.tail = rJL.tail = true;
+    rKL.single = rIK.single = rIL.single = rJK.single = rJL.single = true;
+  }
   double dij[NB], aij[NB];
 #pragma unroll
   for (int mj = 0; mj < NJ; ++mj)
@@ -170,7 +177,10 @@ __device__ __forceinline__ void jk_digest_rows(int base, int ls, int r0, int nr,
       dij[mi + NI * mj] = D[(oI + mi) * n + oJ + mj];
       aij[mi + NI * mj] = 0.0;
     }
-  for (int r = 0; r < nr; ++r) {
+  const bool tuple = live;
+  for (int rr = 0; rr < nr; rr += 1 << lg) {
+    const int r = rr + t < nr ? rr + t : rr;
+    live = tuple && rr + t < nr;
     const int kl = r0 + r, mk = kl % NK, ml = kl / NK;
     const double dkl = D[(oK + mk) * n + oL + ml];
     double djl[NJ], djk[NJ], dil[NI], dik[NI];
@@ -217,7 +227,7 @@ __device__ __forceinline__ void jk_digest_rows(int base, int ls, int r0, int nr,
   for (int mj = 0; mj < NJ; ++mj)
 #pragma unroll
     for (int mi = 0; mi < NI; ++mi)
-      jk_put(live, J, (oI + mi) * n + oJ + mj, 2.0 * w * aij[mi + NI * mj], rIJ);
+      jk_put(tuple, J, (oI + mi) * n + oJ + mj, 2.0 * w * aij[mi + NI * mj], rIJ);
 }
 
 // jk_digest_rows for the compile-time rows [0, NR) (a kernel with one digest
@@ -319,13 +329,14 @@ __device__ __forceinline__ void jk_digest_rows_fixed(int base, int ls, bool live
 }
 
 template <int NI, int NJ, int NK, int NL>
-__device__ __noinline__ void jk_digest_rows_call(int base, int ls, int r0, int nr, bool live,
-                                                 int s0, int s1, int s2, int s3, int o0, int o1,
-                                                 int o2, int o3, const double* __restrict__ D,
+__device__ __noinline__ void jk_digest_rows_call(int base, int ls, int r0, int nr, int t, int lg,
+                                                 bool live, int s0, int s1, int s2, int s3, int o0,
+                                                 int o1, int o2, int o3,
+                                                 const double* __restrict__ D,
                                                  double* __restrict__ J,
                                                  double* __restrict__ K, int nao) {
-  jk_digest_rows<NI, NJ, NK, NL>(base, ls, r0, nr, live, s0, s1, s2, s3, o0, o1, o2, o3, D, J, K,
-                                 nao);
+  jk_digest_rows<NI, NJ, NK, NL>(base, ls, r0, nr, t, lg, live, s0, s1, s2, s3, o0, o1, o2, o3, D,
+                                 J, K, nao);
 }
 
 }  // namespace cx

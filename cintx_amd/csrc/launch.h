@@ -26,6 +26,9 @@ struct Registry {
   KernelInfo k[2][kForms][kMaxL + 1][kMaxL + 1][kMaxL + 1][kMaxL + 1][kVariants];
   // int2e_sph launch shapes with the fused J/K epilogue, FP64 and FP32 forms
   KernelInfo jk[2][kMaxL + 1][kMaxL + 1][kMaxL + 1][kMaxL + 1][kVariants];
+  // a plan's blocks of the class are in the order of surviving primitive
+  // tuples (of primitive counts otherwise)
+  bool by_work[2][kForms][kMaxL + 1][kMaxL + 1][kMaxL + 1][kMaxL + 1];
 };
 
 // Filled by the generated instantiation units.

@@ -565,6 +565,8 @@ struct Bin {
   std::vector<int2> q;
   int64_t out_base = 0;  // element offset of the bin's first block
   int64_t block = 0;     // elements per block (NS * ncomp)
+  // one-lane launches: tuples before lanes_end[k] that take at most 2^k lanes
+  std::array<int64_t, kSplits> lanes_end{};
   // device pointer (inside the plan blob)
   int2* d_q = nullptr;
 };
@@ -784,14 +786,53 @@ static int64_t surviving_prims(const PairSet& S, int bra, int ket, int lij, int 
   return total;
 }
 
+// Lanes per tuple of a one-lane launch over n tuples in ascending order of
+// surviving primitive tuples, `total` in all, of which below(w) have fewer
+// than w: ends[k] is the first tuple that takes more than 2^k lanes.  A tuple is split until its
+// lanes have about `per` primitive tuples each: half of what each of the
+// chip's lanes (one wavefront per SIMD) would get of the whole bin, so that
+// no lane outlasts the rest by much, but four at least, below which a lane's
+// own preparation and the sum over the lanes cost more than they save
+// (two: int3c2e_sph on 24 atoms 1.13 ms instead of 0.92, four-centre lists
+// the same).
+constexpr int64_t kChipLanes = 256 * 4 * 64;
+template <typename F>
+static void split_lanes(int64_t n, int64_t total, F&& below, int64_t* ends) {
+  const int64_t per = std::max<int64_t>(4, total / (2 * kChipLanes));
+  for (int k = 0; k < kSplits; ++k) ends[k] = k == kSplits - 1 ? n : below(per << (k + 1));
+}
+
+// The launch shape of an untuned launch: of a class with a one-lane kernel
+// that kernel, unless the launch is small (its `total` primitive tuples
+// leave lanes idle) and no tuple is long (`most` primitive tuples, which the
+// one-lane kernel spreads over up to 64 lanes and the others walk a few at a
+// time); then the first of the others.  (p p|p p): 1,196 tuples of up to
+// 1,296 primitive tuples 0.08 ms against 0.37 ms; (d p|d s) nabla_i, 1,600
+// tuples of up to 36, 8,600 in all, 0.07 ms against 0.03 ms; int3c2e_sph
+// (d p|d), 233,000 in all, 0.15 ms against 0.08 ms, (p p|d) 0.047 ms against
+// 0.058 ms.  The kernels of several row chunks repeat the recurrences for
+// each, so they pay later.
+static int default_variant(const KernelInfo* ks, int64_t total, int64_t most) {
+  int one = -1, other = -1;
+  for (int v = kVariants - 1; v >= 0; --v) {
+    if (!ks[v].fn) continue;
+    (ks[v].lanes_per_tuple == 1 ? one : other) = v;
+  }
+  if (one < 0 || other < 0) return std::max(0, std::max(one, other));
+  const int64_t fill = ks[one].prims_per_step == 1 ? 40000 : 230000;
+  return (most >= 64 || total >= fill) ? one : other;
+}
+
 static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);
+static int bin_form(const cintx_plan* P, const Bin& b);
 
 // Lay out and upload pairs, bins and offsets in one device blob.
 // Order every bin's tuples by (bra, ket) primitive-pair counts (counting
 // sort), so that the tuples sharing a workgroup of the wide kernels have
-// equal loop trip counts; for a class with a one-lane kernel instead by
-// surviving primitive tuples (stable), so that the lanes of a wavefront,
-// which each walk their own survivors, run equal numbers of iterations.
+// equal loop trip counts; for the classes of Registry::by_work (the one-lane
+// kernels) instead by surviving primitive tuples (stable), so that the lanes
+// of a wavefront, which each walk their own survivors, run equal numbers of
+// iterations and neighbouring tuples can take equal numbers of lanes.
 static void plan_sort_bins(cintx_plan* P) {
   const PairSet& S = P->pairs;
   const FamilyInfo& f = kFam[P->family];
@@ -799,28 +840,27 @@ static void plan_sort_bins(cintx_plan* P) {
   for (size_t bi = 0; bi < P->bins.size(); ++bi) {
     Bin& b = P->bins[bi];
     const int64_t n = (int64_t)b.q.size();
-    auto counting_sort = [&](int K, const std::vector<int>& key, std::vector<int64_t>& pos) {
+    // pos[i]: the place of tuple i; returns the first place of every key
+    auto counting_sort = [&](const std::vector<int>& key, std::vector<int64_t>& pos) {
+      const int K = n ? *std::max_element(key.begin(), key.end()) + 1 : 0;
       std::vector<int64_t> count((size_t)K + 1, 0);
       for (int64_t i = 0; i < n; ++i) ++count[(size_t)key[(size_t)i] + 1];
       for (int k = 0; k < K; ++k) count[k + 1] += count[k];
+      std::vector<int64_t> first = count;
       pos.resize((size_t)n);
       for (int64_t i = 0; i < n; ++i) pos[(size_t)i] = count[(size_t)key[(size_t)i]]++;
+      return first;
     };
-    // first by primitive counts, then (stable) by survivors
     std::vector<int> key((size_t)n);
-    for (int64_t i = 0; i < n; ++i)
-      key[(size_t)i] = std::min(S.np[b.q[i].x], 64) * 65 + std::min(S.np[b.q[i].y], 64);
-    std::vector<int64_t> pos1, pos2;
-    counting_sort(65 * 65, key, pos1);
-    std::vector<int2> by_np((size_t)n);
-    for (int64_t i = 0; i < n; ++i) by_np[(size_t)pos1[(size_t)i]] = b.q[i];
-    bool one_lane = false;
-    if (const KernelInfo* ks = bin_kernels(P, b))
-      for (int v = 0; v < kVariants; ++v)
-        one_lane = one_lane || (ks[v].fn && ks[v].lanes_per_tuple == 1);
-    if (!one_lane) {
-      remap[bi] = pos1;
-      b.q.swap(by_np);
+    std::vector<int64_t>& pos = remap[bi];
+    std::vector<int2> sorted((size_t)n);
+    if (!ctx().reg->by_work[f.deriv][bin_form(P, b)][b.l[0]][b.l[1]][b.l[2]][b.l[3]]) {
+      for (int64_t i = 0; i < n; ++i)
+        key[(size_t)i] = std::min(S.np[b.q[i].x], 64) * 65 + std::min(S.np[b.q[i].y], 64);
+      counting_sort(key, pos);
+      for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos[(size_t)i]] = b.q[(size_t)i];
+      b.q.swap(sorted);
+      b.variant = std::max(b.variant, 0);
       continue;
     }
     // one-lane classes: by survivors alone (stable), so that within equal
@@ -834,10 +874,14 @@ static void plan_sort_bins(cintx_plan* P) {
       key[(size_t)i] = (int)std::min<int64_t>(
           surviving_prims(S, b.q[i].x, b.q[i].y, lij, lkl, f.three, P->expcutoff),
           kSurvCap - 1);
-    counting_sort(kSurvCap, key, pos2);
-    std::vector<int2> sorted((size_t)n);
-    for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos2[(size_t)i]] = b.q[(size_t)i];
-    remap[bi] = pos2;
+    const std::vector<int64_t> first = counting_sort(key, pos);
+    const int64_t most = (int64_t)first.size() - 2;
+    int64_t total = 0;
+    for (int64_t w = 1; w <= most; ++w) total += w * (first[(size_t)w + 1] - first[(size_t)w]);
+    for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos[(size_t)i]] = b.q[(size_t)i];
+    split_lanes(n, total, [&](int64_t w) { return first[(size_t)std::min(w, most + 1)]; },
+                b.lanes_end.data());
+    if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), total, most);
     b.q.swap(sorted);
   }
   for (VQ& v : P->vqs) v.idx = remap[v.bin][(size_t)v.idx];
@@ -1071,7 +1115,7 @@ static void plan_check_kernels(cintx_plan* P) {
     const KernelInfo* ks = bin_kernels(P, b);
     b.generic = (ks[0].fn == nullptr);
     const int v = tuned_slot(P, b);
-    b.variant = (v > 0 && variant_info(P, b, v).fn) ? v : 0;
+    b.variant = (v >= 0 && variant_info(P, b, v).fn) ? v : -1;  // -1: plan_sort_bins chooses
   }
 }
 
@@ -1100,8 +1144,9 @@ struct JkFuse {
 static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
                                const KernelInfo& k, const PairDev& pd, double expcutoff,
                                const int2* d_q, int64_t nq, double* out, int64_t out_base,
-                               int64_t block, double* scratch, unsigned long long* counters,
-                               hipStream_t st, const JkFuse* jk = nullptr) {
+                               int64_t block, const int64_t* lanes_end, double* scratch,
+                               unsigned long long* counters, hipStream_t st,
+                               const JkFuse* jk = nullptr) {
   DevCtx& C = ctx();
   const FamilyInfo& f = kFam[fam];
   const double common_base = (M_PI * M_PI * M_PI) * 2.0 / std::sqrt(M_PI);
@@ -1142,14 +1187,18 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
   }
   // a dispatch holds at most 2^32 - 1 work-items per grid dimension: launch
   // in chunks of at most 2^31 lanes (2^28 tuples for the runtime-class
-  // kernel, whose grid is capped anyway)
+  // kernel, whose grid is capped anyway; 2^24 for the one-lane kernels, of
+  // which a tuple may take 64 lanes)
   const int64_t chunk = generic ? ((int64_t)1 << 28)
-                                : (((int64_t)1 << 31) / std::max(1, k.lanes_per_tuple));
+                        : k.lanes_per_tuple == 1 ? ((int64_t)1 << 24)
+                                                 : (((int64_t)1 << 31) / std::max(1, k.lanes_per_tuple));
   for (int64_t s = 0; s < nq; s += chunk) {
     a.quartets = d_q + s;
     a.out_base = out_base + s * block;
     a.block = block;
     a.nq = std::min(chunk, nq - s);
+    for (int r = 0; r < kSplits; ++r)
+      a.split.end[r] = (int)std::min(a.nq, std::max<int64_t>(0, lanes_end[r] - s));
     hipError_t e;
     // the launch wrappers read the thread's last HIP error after launching;
     // drop any error an earlier, deliberately unchecked call left behind
@@ -1183,7 +1232,7 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   const PairDev pd{P->d_rec, P->d_poff, P->d_pnp, P->d_geo};
   double* scratch = b.generic ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
   launch_bin_kernels(P->family, b.l, b.variant, b.generic, k, pd, P->expcutoff, b.d_q,
-                     (int64_t)b.q.size(), out, b.out_base, b.block, scratch,
+                     (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), scratch,
                      count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
 
@@ -1539,10 +1588,20 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   DevCtx& C = ctx();
   const KernelInfo* ks = C.reg->k[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
   const bool generic = ks[0].fn == nullptr;
+  const double cutoff = fam_expcutoff(fam, env);
+  int64_t total = 0, most = 0;  // surviving primitive tuples
+  for (const int2& v : q) {
+    const int64_t w = surviving_prims(opt ? opt->pairs : local_pairs, v.x, v.y,
+                                      cl[0] + cl[1] + f.deriv, cl[2] + cl[3], f.three, cutoff);
+    total += w;
+    most = std::max(most, w);
+  }
+  int64_t lanes_end[kSplits];  // every block takes the lanes of the longest
+  split_lanes(nq, total, [&](int64_t w) { return most < w ? nq : 0; }, lanes_end);
   int variant = 0;
   if (!generic) {
     const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
-    if (v > 0 && v < kVariants && ks[v].fn) variant = v;
+    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v : default_variant(ks, total, most);
   }
   // natural extents (complex elements for the spinor families)
   int n[4] = {1, 1, 1, 1};
@@ -1581,8 +1640,8 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   HIPCHK(hipMemsetAsync(A + o_cnt, 0, 16, T.stream));
   double* dout = (double*)(A + o_out);
   unsigned long long* dcnt = (unsigned long long*)(A + o_cnt);
-  launch_bin_kernels(fam, cl, variant, generic, ks[variant], pd, fam_expcutoff(fam, env),
-                     (const int2*)(A + o_q), nq, dout, 0, block,
+  launch_bin_kernels(fam, cl, variant, generic, ks[variant], pd, cutoff,
+                     (const int2*)(A + o_q), nq, dout, 0, block, lanes_end,
                      generic ? (double*)(A + o_scr) : nullptr, dcnt, T.stream);
   int d[4] = {n[0], n[1], n[2], n[3]};
   if (dims)

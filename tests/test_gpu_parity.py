@@ -827,3 +827,43 @@ def test_work_counters_match_oracle_model(oracle, variant):
     # class, the oracle in the caller's: the c2s FLOPs differ by the axis order
     assert abs(flops - ref[2]) <= 1e-3 * ref[2]
     p.close()
+
+
+@pytest.mark.parametrize("count", [1, 3, 65, 700])
+def test_lanes_shared_by_a_tuple(oracle, count):
+    """Lists of few and many long contractions, whose tuples take 64 and fewer
+    lanes of the one-lane kernels: odd counts (the last wavefront partly
+    filled), screened-out tuples among them, every output form, and the J/K
+    build that digests split tuples."""
+    mol = M.config(2)
+    rng = np.random.default_rng(90 + count)
+    prims = mol.bas[:, 2]
+    long = np.nonzero(prims >= 4)[0]
+    assert set(int(v) for v in mol.bas[long, 1]) == {0, 1, 2}
+    pick = [tuple(int(s) for s in rng.choice(long, 4)) for _ in range(count)]
+    near = [(t[0], t[0], t[2], t[2]) for t in pick]  # nothing screened: up to 1296 of them
+    for name in ("int2e_sph", "int2e_cart", "int2e_ip1_sph"):
+        check_plan(oracle, name, pick + near, mol)
+    if count == 65:
+        small = M.config(1)
+        p = capi.Plan("int2e_sph", small.atm, small.bas, small.env, screened=(0.0, 1))
+        n = small.nao()
+        D = rng.normal(size=(n, n))
+        D = D + D.T
+        J, K = p.jk(D)
+        shells = range(small.nbas)
+        full = [(i, j, k, l) for l in shells for k in shells for j in shells for i in shells]
+        ref, offs, _ = oracle_blocks(oracle, "int2e_sph", full, small)
+        width = 2 * small.bas[:, 1] + 1
+        off = np.cumsum(width) - width
+        eri = np.zeros((n, n, n, n))
+        for t, o in zip(full, offs):
+            w = [int(width[s]) for s in t]
+            sl = tuple(slice(int(off[s]), int(off[s]) + v) for s, v in zip(t, w))
+            eri[sl] = ref[o:o + int(np.prod(w))].reshape(w[::-1]).transpose(3, 2, 1, 0)
+        Jr = np.einsum("pqrs,rs->pq", eri, D)
+        Kr = np.einsum("pqrs,qs->pr", eri, D)
+        # each of the n^2 terms of an element is within 1e-12 (1 + |eri|)
+        tol = 1e-12 * (1 + np.abs(eri).max()) * np.abs(D).sum()
+        assert np.abs(J - Jr).max() <= tol and np.abs(K - Kr).max() <= tol
+        p.close()
