@@ -125,30 +125,29 @@ def _p2(v):
     return p
 
 
-def register_chunks(deriv, prec, ls, limit=None):
-    """Row chunks for the one-lane path on a class too large for one pass:
-    the g tensor of one root (3*G4 values) and a chunk's FP64 accumulators
-    should fit about 130 doubles of registers (VGPRs plus AGPRs at one wave
-    per SIMD; measured: beyond that the compiler spills tens of KB to scratch
-    and the kernel runs 100x slower).  Every chunk is an unrolled copy of the primitive loop, so at
-    most 3 (more thrash the instruction cache: 6 chunks ran 100x slower);
-    None when that is not enough."""
+def register_doubles(deriv, prec, ls, nch):
+    """Doubles of registers of the one-lane path in nch row chunks: the g
+    tensor of one root (3*G4 values) and a chunk's accumulators (FP32 keeps a
+    per-primitive-tuple partial sum beside each FP64 accumulator)."""
     li, lj, lk, ll = ls
     nc = [(l + 1) * (l + 2) // 2 for l in ls]
     g4 = (li + deriv + 1) * (lj + 1) * (lk + 1) * (ll + 1)
-    gdoubles = 3 * g4 * (8 if prec == 0 else 4) / 8
     nb = nc[0] if deriv else nc[0] * nc[1]
     nrow = nc[0] * nc[1] * nc[2] * nc[3] // nb
-    if gdoubles > 72:
-        return None
-    # FP32 keeps a per-primitive-tuple partial sum beside each FP64 accumulator
-    per_acc = 1.0 if prec == 0 else 1.5
-    # nabla_i holds its factors as well: from 108 doubles on it spilled 0.4 to
-    # 1.2 KB per lane and ran 20 to 50 times slower
-    limit = limit or (105 if deriv else 130)
-    for nch in (2, 3):
-        rpc = -(-nrow // nch)
-        if gdoubles + per_acc * rpc * nb * (3 if deriv else 1) <= limit:
+    return (3 * g4 if prec == 0 else 1.5 * g4) + \
+        (1.0 if prec == 0 else 1.5) * -(-nrow // nch) * nb * (3 if deriv else 1)
+
+
+def register_chunks(deriv, prec, ls):
+    """Row chunks of the one-lane path: the fewest (each repeats the roots and
+    the recurrences: (d p|d s) of a 64-atom molecule takes 2.06 ms in one
+    chunk and 2.81 ms in two) whose registers fit: up to 200 doubles compile
+    without scratch to at most 481 of the 512 VGPRs and AGPRs of one wave per
+    SIMD, 210 and more spill.  Every chunk is an unrolled copy of the primitive loop, so at
+    most 3 (more thrash the instruction cache: 6 chunks ran 100x slower);
+    None when that is not enough."""
+    for nch in (1, 2, 3):
+        if register_doubles(deriv, prec, ls, nch) <= 200:
             return nch
     return None
 
@@ -163,7 +162,9 @@ def by_work(deriv, prec, ls):
     ne = nc[0] * nc[1] * nc[2] * nc[3] * (3 if deriv else 1)
     if is_high_l(deriv, ls):
         return ne <= 81 and not needs_pb(ls) and (deriv == 1 or nc[0] * nc[1] <= 36)
-    return ne <= 81 or register_chunks(deriv, prec, ls, limit=130) is not None
+    g4 = (ls[0] + deriv + 1) * (ls[1] + 1) * (ls[2] + 1) * (ls[3] + 1)
+    return ne <= 81 or ((g4 <= 24 if prec == 0 else g4 <= 48) and any(
+        register_doubles(deriv, prec, ls, nch) <= 130 for nch in (2, 3)))
 
 
 def variants(deriv, prec, ls):
@@ -209,7 +210,7 @@ def variants(deriv, prec, ls):
     # register kernels then spill and run 1-7x slower, so it is not offered)
     if ne <= 27:
         cands.insert(0, (1, 1))
-    elif ne <= 81:
+    elif ne <= 81 and is_high_l(deriv, ls):
         cands.insert(3, (1, 1))
     elif not is_high_l(deriv, ls):
         # (f/g classes: no chunked one-lane variant; with the promoted-alloca
@@ -239,27 +240,29 @@ def variants(deriv, prec, ls):
     return out[:6]
 
 
-# Translation units of the chunked one-lane variants are compiled with larger
-# alloca-to-register limits: their g tensor (up to 81 doubles) is indexed with
-# compile-time constants only after full unrolling, and the default limits
-# leave it in scratch memory.
+# Translation units of the larger one-lane variants are compiled with larger
+# unrolling and alloca-to-register limits: their g tensor and accumulators (up
+# to 200 doubles) are indexed with compile-time constants only after full
+# unrolling, and the default limits leave the loop over more than about 80
+# elements rolled and the arrays in scratch memory (100 KB per lane).
 CHUNK_FLAGS = ["-mllvm", "-amdgpu-promote-alloca-to-vector-limit=4096",
                "-mllvm", "-amdgpu-promote-alloca-to-vector-max-regs=512",
-               "-mllvm", "-amdgpu-promote-alloca-to-vector-vgpr-ratio=1"]
+               "-mllvm", "-amdgpu-promote-alloca-to-vector-vgpr-ratio=1",
+               "-mllvm", "-pragma-unroll-threshold=200000"]
 
 
-def generate(nparts=24, nchunkparts=12):
+def generate(nparts=24, nchunkparts=24):
     os.makedirs(GEN, exist_ok=True)
     classes = class_sets()
     plain, chunked = [], []
     for deriv, prec, ls in classes:
         for v, (tt, pp) in enumerate(variants(deriv, prec, ls)):
-            (chunked if (tt == 1 and (pp & 255) > 1) else plain).append((deriv, prec, ls, v, tt, pp))
+            large = tt == 1 and register_doubles(deriv, prec, ls, pp & 255) > 60
+            (chunked if large else plain).append((deriv, prec, ls, v, tt, pp))
             # the same launch shape with the fused J/K epilogue (PP bit 12):
             # int2e_sph classes in FP64 and FP32 (not the f/g classes)
             if deriv == 0 and prec in (0, 1) and not is_high_l(deriv, ls):
-                (chunked if (tt == 1 and (pp & 255) > 1) else plain).append(
-                    (deriv, prec, ls, v, tt, pp | 4096))
+                (chunked if large else plain).append((deriv, prec, ls, v, tt, pp | 4096))
     parts = [plain[i::nparts] for i in range(nparts)]
     parts += [chunked[i::nchunkparts] for i in range(nchunkparts)]
     nparts = len(parts)

@@ -519,6 +519,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   const int64_t q = REG ? (int64_t)sb.first + slot : (int64_t)heavy_first_block() * Q + slot;
   const bool active = q < (REG ? (int64_t)sb.end : a.nq);
   const int2 pq = a.quartets[active ? q : 0];
+  const int64_t place = a.place && active ? a.place[q] : q;  // block of the output
   const int boff = a.pair_off[pq.x];
   const int koff = a.pair_off[pq.y];
   const double* gb = a.pair_geo + 8 * (size_t)pq.x;
@@ -897,7 +898,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
         }
       }
       if (!active || t != 0) continue;
-      double* o = a.out + a.out_base + q * a.block + comp * a.st_comp;
+      double* o = a.out + a.out_base + place * a.block + comp * a.st_comp;
 #pragma unroll
       for (int ml = 0; ml < NSL; ++ml)
 #pragma unroll
@@ -1238,7 +1239,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
       fused = true;
     }
     if (active && !fused) {
-      double* o = a.out + a.out_base + q * a.block + comp * a.st_comp;
+      double* o = a.out + a.out_base + place * a.block + comp * a.st_comp;
       for (int e = t; e < NS; e += T) {
         int mi = e % NSI, e1 = e / NSI;
         int mj = e1 % NSJ, e2 = e1 / NSJ;

@@ -567,8 +567,11 @@ struct Bin {
   int64_t block = 0;     // elements per block (NS * ncomp)
   // one-lane launches: tuples before lanes_end[k] that take at most 2^k lanes
   std::array<int64_t, kSplits> lanes_end{};
-  // device pointer (inside the plan blob)
+  // block number of every tuple of q, where that is not its own number
+  std::vector<int> place;
+  // device pointers (inside the plan blob)
   int2* d_q = nullptr;
+  int* d_place = nullptr;
 };
 
 struct VQ {  // one virtual (segmented) tuple of a caller tuple
@@ -802,37 +805,46 @@ static void split_lanes(int64_t n, int64_t total, F&& below, int64_t* ends) {
   for (int k = 0; k < kSplits; ++k) ends[k] = k == kSplits - 1 ? n : below(per << (k + 1));
 }
 
-// The launch shape of an untuned launch: of a class with a one-lane kernel
-// that kernel, unless the launch is small (its `total` primitive tuples
-// leave lanes idle) and no tuple is long (`most` primitive tuples, which the
-// one-lane kernel spreads over up to 64 lanes and the others walk a few at a
-// time); then the first of the others.  (p p|p p): 1,196 tuples of up to
-// 1,296 primitive tuples 0.08 ms against 0.37 ms; (d p|d s) nabla_i, 1,600
-// tuples of up to 36, 8,600 in all, 0.07 ms against 0.03 ms; int3c2e_sph
-// (d p|d), 233,000 in all, 0.15 ms against 0.08 ms, (p p|d) 0.047 ms against
-// 0.058 ms.  The kernels of several row chunks repeat the recurrences for
-// each, so they pay later.
-static int default_variant(const KernelInfo* ks, int64_t total, int64_t most) {
+// The launch shape of an untuned launch of class l: of a class with a
+// one-lane kernel that kernel, unless the launch is small (its `total`
+// primitive tuples leave lanes idle) and no tuple is long (`most` primitive
+// tuples, which the one-lane kernel spreads over up to 64 lanes and the
+// others walk a few at a time); then the first of the others.  (p p|p p),
+// 1,196 tuples of up to 1,296 primitive tuples: 0.08 ms against 0.37 ms.
+// With at most 36 primitive tuples each, the line lies higher the longer a
+// primitive tuple takes one lane, which follows its registers (g tensor and
+// accumulators) times its row chunks: int3c2e_sph (p p|d), 234,000 primitive
+// tuples, 0.038 ms against 0.061 ms; (d p|d), 233,000, 0.067 against 0.084;
+// (d d|p), 87,000, 0.053 against 0.040; (d p|f), 175,000 in two chunks, 0.17
+// against 0.10; (d p|p) nabla_i, 13,000 in two, 0.07 against 0.03.
+static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_t total,
+                           int64_t most) {
   int one = -1, other = -1;
   for (int v = kVariants - 1; v >= 0; --v) {
     if (!ks[v].fn) continue;
     (ks[v].lanes_per_tuple == 1 ? one : other) = v;
   }
   if (one < 0 || other < 0) return std::max(0, std::max(one, other));
-  const int64_t fill = ks[one].prims_per_step == 1 ? 40000 : 230000;
-  return (most >= 64 || total >= fill) ? one : other;
+  const int64_t nch = ks[one].prims_per_step;
+  const int64_t g = 3LL * (l[0] + deriv + 1) * (l[1] + 1) * (l[2] + 1) * (l[3] + 1);
+  const int64_t acc = (int64_t)ncart(l[0]) * ncart(l[1]) * ncart(l[2]) * ncart(l[3]) *
+                      (deriv ? 3 : 1) / nch;
+  return (most >= 64 || total >= 700 * (g + acc) * nch) ? one : other;
 }
 
 static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);
+static const KernelInfo& variant_info(const cintx_plan* P, const Bin& b, int v);
 static int bin_form(const cintx_plan* P, const Bin& b);
 
-// Lay out and upload pairs, bins and offsets in one device blob.
-// Order every bin's tuples by (bra, ket) primitive-pair counts (counting
-// sort), so that the tuples sharing a workgroup of the wide kernels have
-// equal loop trip counts; for the classes of Registry::by_work (the one-lane
-// kernels) instead by surviving primitive tuples (stable), so that the lanes
-// of a wavefront, which each walk their own survivors, run equal numbers of
-// iterations and neighbouring tuples can take equal numbers of lanes.
+// A bin's blocks are placed by (bra, ket) primitive-pair counts (counting
+// sort), or for the classes of Registry::by_work by surviving primitive
+// tuples (stable).  Its tuples are listed in that order, except that a class
+// with a one-lane kernel always lists them by surviving primitive tuples, so
+// that the lanes of a wavefront, which each walk their own survivors, run
+// equal numbers of iterations and neighbouring tuples take equal numbers of
+// lanes; `place` then holds the block of every tuple.  (The wide kernels'
+// tuples share a workgroup best with equal loop counts, which either order
+// gives them.)
 static void plan_sort_bins(cintx_plan* P) {
   const PairSet& S = P->pairs;
   const FamilyInfo& f = kFam[P->family];
@@ -852,37 +864,50 @@ static void plan_sort_bins(cintx_plan* P) {
       return first;
     };
     std::vector<int> key((size_t)n);
-    std::vector<int64_t>& pos = remap[bi];
-    std::vector<int2> sorted((size_t)n);
-    if (!ctx().reg->by_work[f.deriv][bin_form(P, b)][b.l[0]][b.l[1]][b.l[2]][b.l[3]]) {
+    std::vector<int64_t>& pos = remap[bi];  // blocks
+    std::vector<int64_t> by_work;           // places in the list, where not the blocks
+    const bool placed_by_work =
+        ctx().reg->by_work[f.deriv][bin_form(P, b)][b.l[0]][b.l[1]][b.l[2]][b.l[3]];
+    bool one_lane = false;
+    for (int v = 0; v < 2 * kVariants; ++v) {
+      const KernelInfo& k = variant_info(P, b, v);
+      one_lane = one_lane || (k.fn && k.lanes_per_tuple == 1);
+    }
+    if (!placed_by_work) {
       for (int64_t i = 0; i < n; ++i)
         key[(size_t)i] = std::min(S.np[b.q[i].x], 64) * 65 + std::min(S.np[b.q[i].y], 64);
       counting_sort(key, pos);
-      for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos[(size_t)i]] = b.q[(size_t)i];
-      b.q.swap(sorted);
-      b.variant = std::max(b.variant, 0);
-      continue;
     }
-    // one-lane classes: by survivors alone (stable), so that within equal
-    // survivor counts the enumeration's bra-major order stays and
-    // neighbouring lanes often share their bra pair (the fused J/K sums
-    // such lanes before its atomics); a lane walks its survivors only, so
-    // the primitive counts do not set its trip count
-    const int lij = b.l[0] + b.l[1] + f.deriv, lkl = b.l[2] + b.l[3];
-    constexpr int kSurvCap = 1 << 16;
-    for (int64_t i = 0; i < n; ++i)
-      key[(size_t)i] = (int)std::min<int64_t>(
-          surviving_prims(S, b.q[i].x, b.q[i].y, lij, lkl, f.three, P->expcutoff),
-          kSurvCap - 1);
-    const std::vector<int64_t> first = counting_sort(key, pos);
-    const int64_t most = (int64_t)first.size() - 2;
-    int64_t total = 0;
-    for (int64_t w = 1; w <= most; ++w) total += w * (first[(size_t)w + 1] - first[(size_t)w]);
-    for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos[(size_t)i]] = b.q[(size_t)i];
-    split_lanes(n, total, [&](int64_t w) { return first[(size_t)std::min(w, most + 1)]; },
-                b.lanes_end.data());
-    if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), total, most);
+    if (placed_by_work || one_lane) {
+      // by survivors alone, so that within equal survivor counts the
+      // enumeration's bra-major order stays and neighbouring lanes often
+      // share their bra pair (the fused J/K sums such lanes before its
+      // atomics); a lane walks its survivors only, so the primitive counts do
+      // not set its trip count
+      const int lij = b.l[0] + b.l[1] + f.deriv, lkl = b.l[2] + b.l[3];
+      constexpr int kSurvCap = 1 << 16;
+      for (int64_t i = 0; i < n; ++i)
+        key[(size_t)i] = (int)std::min<int64_t>(
+            surviving_prims(S, b.q[i].x, b.q[i].y, lij, lkl, f.three, P->expcutoff),
+            kSurvCap - 1);
+      const std::vector<int64_t> first = counting_sort(key, placed_by_work ? pos : by_work);
+      const int64_t most = (int64_t)first.size() - 2;
+      int64_t total = 0;
+      for (int64_t w = 1; w <= most; ++w) total += w * (first[(size_t)w + 1] - first[(size_t)w]);
+      split_lanes(n, total, [&](int64_t w) { return first[(size_t)std::min(w, most + 1)]; },
+                  b.lanes_end.data());
+      if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, total, most);
+    }
+    b.variant = std::max(b.variant, 0);
+    const std::vector<int64_t>& at = by_work.empty() ? pos : by_work;
+    std::vector<int2> sorted((size_t)n);
+    for (int64_t i = 0; i < n; ++i) sorted[(size_t)at[(size_t)i]] = b.q[(size_t)i];
     b.q.swap(sorted);
+    if (!by_work.empty()) {
+      if (n > INT32_MAX) fail(CINTX_STATUS_MEMORY_LIMIT_EXCEEDED, "too many tuples of one class");
+      b.place.resize((size_t)n);
+      for (int64_t i = 0; i < n; ++i) b.place[(size_t)at[(size_t)i]] = (int)pos[(size_t)i];
+    }
   }
   for (VQ& v : P->vqs) v.idx = remap[v.bin][(size_t)v.idx];
 }
@@ -929,6 +954,7 @@ static int spinor_grid(int64_t njobs, int64_t slice, size_t budget) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({njobs, fit, (int64_t)2048}));
 }
 
+// Lay out and upload pairs, bins and offsets in one device blob.
 static void plan_upload(cintx_plan* P) {
   DevCtx& C = ctx();
   const FamilyInfo& fam = kFam[P->family];
@@ -972,8 +998,11 @@ static void plan_upload(cintx_plan* P) {
   };
   size_t o_rec = take(npp * 64);
   size_t o_poff = take(npair * 4), o_pnp = take(npair * 4), o_geo = take(npair * 64);
-  std::vector<size_t> o_q(P->bins.size());
-  for (size_t i = 0; i < P->bins.size(); ++i) o_q[i] = take(P->bins[i].q.size() * sizeof(int2));
+  std::vector<size_t> o_q(P->bins.size()), o_place(P->bins.size());
+  for (size_t i = 0; i < P->bins.size(); ++i) {
+    o_q[i] = take(P->bins[i].q.size() * sizeof(int2));
+    o_place[i] = take(P->bins[i].place.size() * sizeof(int));
+  }
   size_t o_cnt = take(P->bins.size() * 2 * 8 + 8);
   const int nbas = P->basis.nbas;
   size_t o_ao = take((size_t)nbas * 4), o_l = take((size_t)nbas * 4),
@@ -1039,6 +1068,8 @@ static void plan_upload(cintx_plan* P) {
     Bin& b = P->bins[i];
     put(o_q[i], b.q.data(), b.q.size() * sizeof(int2));
     b.d_q = (int2*)(P->blob + o_q[i]);
+    put(o_place[i], b.place.data(), b.place.size() * sizeof(int));
+    b.d_place = b.place.empty() ? nullptr : (int*)(P->blob + o_place[i]);
   }
   HIPCHK(hipMemcpyAsync(P->blob, h.data(), host_bytes, hipMemcpyHostToDevice, C.stream));
   if (!jobs.empty())
@@ -1143,8 +1174,8 @@ struct JkFuse {
 
 static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
                                const KernelInfo& k, const PairDev& pd, double expcutoff,
-                               const int2* d_q, int64_t nq, double* out, int64_t out_base,
-                               int64_t block, const int64_t* lanes_end, double* scratch,
+                               const int2* d_q, const int* d_place, int64_t nq, double* out,
+                               int64_t out_base, int64_t block, const int64_t* lanes_end, double* scratch,
                                unsigned long long* counters, hipStream_t st,
                                const JkFuse* jk = nullptr) {
   DevCtx& C = ctx();
@@ -1194,7 +1225,8 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
                                                  : (((int64_t)1 << 31) / std::max(1, k.lanes_per_tuple));
   for (int64_t s = 0; s < nq; s += chunk) {
     a.quartets = d_q + s;
-    a.out_base = out_base + s * block;
+    a.place = d_place ? d_place + s : nullptr;
+    a.out_base = out_base + (d_place ? 0 : s * block);
     a.block = block;
     a.nq = std::min(chunk, nq - s);
     for (int r = 0; r < kSplits; ++r)
@@ -1232,7 +1264,7 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   const PairDev pd{P->d_rec, P->d_poff, P->d_pnp, P->d_geo};
   double* scratch = b.generic ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
   launch_bin_kernels(P->family, b.l, b.variant, b.generic, k, pd, P->expcutoff, b.d_q,
-                     (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), scratch,
+                     b.d_place, (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), scratch,
                      count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
 
@@ -1601,7 +1633,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   int variant = 0;
   if (!generic) {
     const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
-    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v : default_variant(ks, total, most);
+    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v : default_variant(ks, cl, f.deriv, total, most);
   }
   // natural extents (complex elements for the spinor families)
   int n[4] = {1, 1, 1, 1};
@@ -1641,7 +1673,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   double* dout = (double*)(A + o_out);
   unsigned long long* dcnt = (unsigned long long*)(A + o_cnt);
   launch_bin_kernels(fam, cl, variant, generic, ks[variant], pd, cutoff,
-                     (const int2*)(A + o_q), nq, dout, 0, block, lanes_end,
+                     (const int2*)(A + o_q), nullptr, nq, dout, 0, block, lanes_end,
                      generic ? (double*)(A + o_scr) : nullptr, dcnt, T.stream);
   int d[4] = {n[0], n[1], n[2], n[3]};
   if (dims)
@@ -2613,8 +2645,7 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
         for (const SP& s : sp) qof[((uint64_t)s.a << 32) | (uint32_t)s.b] = qabs[(size_t)s.id];
         // FP32 without packed math issues at the FP64 rate on CDNA4: the FP32
         // recurrences pay only in classes that must share g through LDS (half
-        // the LDS bytes and registers); classes with a one-lane register
-        // kernel are faster in FP64, so they stay FP64
+        // the LDS bytes and registers), which are those not placed by work
         auto fp32_pays = [&](const int* sh) {
           int la = B.l[sh[0]], lb = B.l[sh[1]], lc = B.l[sh[2]], ld = B.l[sh[3]];
           if (lc > la || (lc == la && ld > lb)) {
@@ -2622,11 +2653,8 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
             std::swap(lb, ld);
           }
           if (la > kMaxL || lb > kMaxL || lc > kMaxL || ld > kMaxL) return false;
-          const KernelInfo* k64 = ctx().reg->k[0][0][la][lb][lc][ld];
-          if (!ctx().reg->k[0][1][la][lb][lc][ld][0].fn) return false;  // no FP32 build
-          for (int v = 0; v < kVariants; ++v)
-            if (k64[v].fn && k64[v].lanes_per_tuple == 1) return false;
-          return true;
+          return ctx().reg->k[0][1][la][lb][lc][ld][0].fn != nullptr &&
+                 !ctx().reg->by_work[0][0][la][lb][lc][ld];
         };
         for (int64_t t = 0; t < nt; ++t) {
           double b = qof[((uint64_t)tuples[4 * t] << 32) | (uint32_t)tuples[4 * t + 1]] *
