@@ -47,6 +47,9 @@ constexpr int kSplits = 7;
 struct LaneSplit {
   int end[kSplits];
 };
+constexpr int64_t kGenericGrid = 1024;  // workgroups of a large runtime-class launch
+constexpr int64_t kGenFew = 2048;  // fewer tuples: several workgroups may share one
+constexpr int64_t kGenFill = 512;  // workgroups that fill the chip: 256 CUs, 2 each
 constexpr int kOneLaneBlock = 256;  // lanes of a one-lane kernel's workgroup
 __host__ __device__ constexpr int split_blocks(int n, int lg) {
   return (int)((((int64_t)n << lg) + kOneLaneBlock - 1) / kOneLaneBlock);

@@ -31,8 +31,9 @@ namespace cx {
 
 hipError_t launch_rys_eval(const RysTable& tab, int n, const double* x, int64_t nx, double* u,
                            double* w, hipStream_t s);
-hipError_t launch_generic(const EriArgs& a, const int* l, int deriv, int grid, hipStream_t s);
-int64_t generic_scratch_per_block(const int* l, int deriv);
+hipError_t launch_generic(const EriArgs& a, const int* l, int deriv, int64_t most,
+                          hipStream_t s);
+int64_t generic_scratch(const int* l, int deriv, int64_t nq, int64_t most);
 hipError_t mlp_train_device(const RysTable& tab, float* prm, int64_t nsamples, int epochs,
                             int batch, float lr, uint64_t seed, double* final_loss,
                             hipStream_t st);
@@ -48,12 +49,11 @@ hipError_t launch_jk_sym_copy(const double* src, double* dst, int n, hipStream_t
 hipError_t jk_scratch_address(double** ptr);
 size_t jk_scratch_bytes();
 hipError_t launch_jk_digest(const double* eri, int64_t out_base, int64_t block, const int2* q,
-                            int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
+                            const int* place, int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
                             const double* D, double* J, double* K, int nao, hipStream_t s);
 hipError_t launch_spinor(const SpinorJob* jobs, int64_t njobs, const double* cart, double* out,
                          const double* tab, const double* c2s, double* scratch, int64_t slice,
                          int grid, bool four, hipStream_t s);
-static constexpr int kGenericGrid = 1024;
 
 // ------------------------------------------------------------------
 // Errors: fail-closed, typed, thread-local last error.
@@ -561,6 +561,9 @@ struct Bin {
   double prim_tuples = 0;       // from the last work count
   double flops = 0;
   bool generic = false;  // no compile-time instantiation: runtime-class kernel
+  bool small = false;    // may run the runtime-class kernel, its default
+  int64_t most = 0;      // primitive tuples of its longest tuple (runtime-class launches)
+  bool runtime_class() const;  // the launch shape in use is the runtime-class kernel
   int variant = 0;       // class-kernel variant (launch shape) in use
   std::vector<int2> q;
   int64_t out_base = 0;  // element offset of the bin's first block
@@ -805,31 +808,52 @@ static void split_lanes(int64_t n, int64_t total, F&& below, int64_t* ends) {
   for (int k = 0; k < kSplits; ++k) ends[k] = k == kSplits - 1 ? n : below(per << (k + 1));
 }
 
-// The launch shape of an untuned launch of class l: of a class with a
-// one-lane kernel that kernel, unless the launch is small (its `total`
-// primitive tuples leave lanes idle) and no tuple is long (`most` primitive
-// tuples, which the one-lane kernel spreads over up to 64 lanes and the
-// others walk a few at a time); then the first of the others.  (p p|p p),
-// 1,196 tuples of up to 1,296 primitive tuples: 0.08 ms against 0.37 ms.
-// With at most 36 primitive tuples each, the line lies higher the longer a
-// primitive tuple takes one lane, which follows its registers (g tensor and
-// accumulators) times its row chunks: int3c2e_sph (p p|d), 234,000 primitive
-// tuples, 0.038 ms against 0.061 ms; (d p|d), 233,000, 0.067 against 0.084;
-// (d d|p), 87,000, 0.053 against 0.040; (d p|f), 175,000 in two chunks, 0.17
-// against 0.10; (d p|p) nabla_i, 13,000 in two, 0.07 against 0.03.
-static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_t total,
-                           int64_t most) {
+// Number of the runtime-class kernel among a bin's launch shapes: beyond the
+// compiled variants and (FP32 bins) their FP64 instantiations.
+constexpr int kRuntimeClass = 2 * kVariants;
+inline bool Bin::runtime_class() const { return generic || variant == kRuntimeClass; }
+
+// The launch shape of an untuned launch of class l: `total` primitive tuples,
+// `most` of them in the longest tuple.
+//
+// Large launches of a class with a one-lane kernel take that kernel.  With
+// short tuples (at most 36 primitive tuples, say) the line lies higher the
+// longer a primitive tuple takes one lane, which follows its registers (g
+// tensor and accumulators) times its row chunks: int3c2e_sph (p p|d), 234,000
+// primitive tuples, 0.038 ms against 0.061 ms in the wide kernel; (d p|d),
+// 233,000, 0.067 against 0.084; (d d|p), 87,000, 0.053 against 0.040; (d p|f),
+// 175,000 in two chunks, 0.17 against 0.10; (d p|p) nabla_i, 13,000 in two,
+// 0.07 against 0.03.
+//
+// Long tuples are what the wide kernels, which walk a tuple a few primitive
+// tuples at a time, are worst at; the one-lane kernels spread one over up to
+// 64 lanes and the runtime-class kernel over many workgroups.  (p p|p p),
+// 1,196 tuples of up to 1,296, 112,000 in all: 0.08 ms one-lane, 0.37 ms wide,
+// 0.22 ms runtime-class.  The runtime-class kernel is the fastest of the three
+// where a launch is small and the one-lane kernel large or missing: (d p|p p),
+// 150 tuples, 30,000 in all, 0.12 ms against 0.19 ms one-lane; (d d|d p), 400
+// tuples, 56,000, 0.31 ms against 0.43 ms wide; (d p|d p), 820 tuples, 80,000,
+// equal.  It keeps more of the chip busy for it, so beside the other bins of a
+// plan it pays at a quarter of those sizes: int2e_ip1_sph, 300,000 tuples of
+// 18 atoms, 4.3 ms with the lines below and 5.8 ms with four times as large
+// ones; the integrals of 3 atoms 0.8 ms, and 2.9 ms without it.
+static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_t nq,
+                           int64_t total, int64_t most) {
   int one = -1, other = -1;
   for (int v = kVariants - 1; v >= 0; --v) {
     if (!ks[v].fn) continue;
     (ks[v].lanes_per_tuple == 1 ? one : other) = v;
   }
-  if (one < 0 || other < 0) return std::max(0, std::max(one, other));
+  const bool is_long = most >= 64;
+  const bool splits = nq < kGenFew;  // the runtime-class kernel's tuples go to several workgroups
+  if (one < 0) return is_long && splits && total < 20000 ? kRuntimeClass : std::max(other, 0);
   const int64_t nch = ks[one].prims_per_step;
   const int64_t g = 3LL * (l[0] + deriv + 1) * (l[1] + 1) * (l[2] + 1) * (l[3] + 1);
   const int64_t acc = (int64_t)ncart(l[0]) * ncart(l[1]) * ncart(l[2]) * ncart(l[3]) *
                       (deriv ? 3 : 1) / nch;
-  return (most >= 64 || total >= 700 * (g + acc) * nch) ? one : other;
+  const int64_t size = (g + acc) * nch;
+  if (is_long) return size >= 125 && splits && total < 75 * size ? kRuntimeClass : one;
+  return other < 0 || total >= 700 * size ? one : other;
 }
 
 static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);
@@ -878,6 +902,16 @@ static void plan_sort_bins(cintx_plan* P) {
         key[(size_t)i] = std::min(S.np[b.q[i].x], 64) * 65 + std::min(S.np[b.q[i].y], 64);
       counting_sort(key, pos);
     }
+    if (!placed_by_work && !one_lane && !b.generic && b.variant < 0) {
+      int64_t total = 0, most = 0;
+      for (const int2& v : b.q) {
+        const int64_t w = surviving_prims(S, v.x, v.y, b.l[0] + b.l[1] + f.deriv, b.l[2] + b.l[3],
+                                          f.three, P->expcutoff);
+        total += w;
+        most = std::max(most, w);
+      }
+      b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
+    }
     if (placed_by_work || one_lane) {
       // by survivors alone, so that within equal survivor counts the
       // enumeration's bra-major order stays and neighbouring lanes often
@@ -896,9 +930,10 @@ static void plan_sort_bins(cintx_plan* P) {
       for (int64_t w = 1; w <= most; ++w) total += w * (first[(size_t)w + 1] - first[(size_t)w]);
       split_lanes(n, total, [&](int64_t w) { return first[(size_t)std::min(w, most + 1)]; },
                   b.lanes_end.data());
-      if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, total, most);
+      if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
     }
     b.variant = std::max(b.variant, 0);
+    b.small = b.variant == kRuntimeClass;
     const std::vector<int64_t>& at = by_work.empty() ? pos : by_work;
     std::vector<int2> sorted((size_t)n);
     for (int64_t i = 0; i < n; ++i) sorted[(size_t)at[(size_t)i]] = b.q[(size_t)i];
@@ -1009,16 +1044,18 @@ static void plan_upload(cintx_plan* P) {
          o_psh = take(npair * sizeof(int2));
   int64_t scratch = 0;
   for (auto& b : P->bins)
-    if (b.generic) {
-      int64_t grid = std::min<int64_t>((int64_t)b.q.size(), kGenericGrid);
-      scratch = std::max(scratch, grid * generic_scratch_per_block(b.l, kFam[P->family].deriv));
+    if (b.generic || b.small) {
+      for (const int2& v : b.q)
+        b.most = std::max<int64_t>(b.most, (int64_t)S.np[v.x] * S.np[v.y]);
+      scratch = std::max(scratch, generic_scratch(b.l, kFam[P->family].deriv,
+                                                  (int64_t)b.q.size(), b.most));
     }
   size_t o_out = take((size_t)P->total * 8);
   // one workspace per graph chain that runs runtime-class bins (so those of
   // different chains run concurrently): as many slices as such bins, up to
   // the chain count, fewer when that would pass 8 GiB
   int ngeneric = 0;
-  for (auto& b : P->bins) ngeneric += b.generic ? 1 : 0;
+  for (auto& b : P->bins) ngeneric += b.generic || b.small ? 1 : 0;
   P->scratch_chains = 1;
   while (P->scratch_chains < kChains && 2 * P->scratch_chains <= ngeneric &&
          (size_t)scratch * 8 * (size_t)(2 * P->scratch_chains) <= ((size_t)8 << 30))
@@ -1161,7 +1198,8 @@ struct PairDev {
 // One class bin's launches: nq tuples d_q[0..nq) of class l (canonical
 // slots) and form prec, blocks of `block` elements written from out_base.
 // Variant `k` of the compiled class kernels, or the runtime-class kernel
-// (generic) with `scratch` of kGenericGrid slices.
+// (generic, tuples of at most `most` primitive tuples) with `scratch` of
+// generic_scratch doubles.
 // Fused J/K of a launch: the class kernel digests its blocks into J/K.
 struct JkFuse {
   const double* D;
@@ -1175,7 +1213,8 @@ struct JkFuse {
 static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
                                const KernelInfo& k, const PairDev& pd, double expcutoff,
                                const int2* d_q, const int* d_place, int64_t nq, double* out,
-                               int64_t out_base, int64_t block, const int64_t* lanes_end, double* scratch,
+                               int64_t out_base, int64_t block, const int64_t* lanes_end,
+                               int64_t most, double* scratch,
                                unsigned long long* counters, hipStream_t st,
                                const JkFuse* jk = nullptr) {
   DevCtx& C = ctx();
@@ -1217,10 +1256,10 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
     a.nao = jk->nao;
   }
   // a dispatch holds at most 2^32 - 1 work-items per grid dimension: launch
-  // in chunks of at most 2^31 lanes (2^28 tuples for the runtime-class
+  // in chunks of at most 2^31 lanes (all tuples for the runtime-class
   // kernel, whose grid is capped anyway; 2^24 for the one-lane kernels, of
   // which a tuple may take 64 lanes)
-  const int64_t chunk = generic ? ((int64_t)1 << 28)
+  const int64_t chunk = generic ? std::max<int64_t>(nq, 1)
                         : k.lanes_per_tuple == 1 ? ((int64_t)1 << 24)
                                                  : (((int64_t)1 << 31) / std::max(1, k.lanes_per_tuple));
   for (int64_t s = 0; s < nq; s += chunk) {
@@ -1236,8 +1275,7 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
     // drop any error an earlier, deliberately unchecked call left behind
     (void)hipGetLastError();
     if (generic) {
-      int grid = (int)std::min<int64_t>(a.nq, kGenericGrid);
-      e = launch_generic(a, l, f.deriv, grid, st);
+      e = launch_generic(a, l, f.deriv, most, st);
     } else {
       e = k.fn(a, st);
     }
@@ -1262,9 +1300,10 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   if (kFam[P->family].spinor) out = P->d_cart;  // the transform reads them from there
   const KernelInfo& k = jk ? variant_info_jk(P, b, b.variant) : variant_info(P, b, b.variant);
   const PairDev pd{P->d_rec, P->d_poff, P->d_pnp, P->d_geo};
-  double* scratch = b.generic ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
-  launch_bin_kernels(P->family, b.l, b.variant, b.generic, k, pd, P->expcutoff, b.d_q,
-                     b.d_place, (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), scratch,
+  double* scratch = b.runtime_class() ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
+  launch_bin_kernels(P->family, b.l, b.variant, b.runtime_class(), k, pd, P->expcutoff, b.d_q,
+                     b.d_place, (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(),
+                     b.most, scratch,
                      count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
 
@@ -1619,7 +1658,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   // runtime-class kernel
   DevCtx& C = ctx();
   const KernelInfo* ks = C.reg->k[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
-  const bool generic = ks[0].fn == nullptr;
+  bool generic = ks[0].fn == nullptr;
   const double cutoff = fam_expcutoff(fam, env);
   int64_t total = 0, most = 0;  // surviving primitive tuples
   for (const int2& v : q) {
@@ -1633,7 +1672,12 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   int variant = 0;
   if (!generic) {
     const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
-    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v : default_variant(ks, cl, f.deriv, total, most);
+    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v
+                                                    : default_variant(ks, cl, f.deriv, nq, total, most);
+    if (variant == kRuntimeClass) {
+      generic = true;
+      variant = 0;
+    }
   }
   // natural extents (complex elements for the spinor families)
   int n[4] = {1, 1, 1, 1};
@@ -1659,8 +1703,12 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   const size_t o_q = pbytes, o_out = o_q + align256(nq * sizeof(int2));
   const size_t o_cnt = o_out + align256(nq * block * 8);
   const size_t o_scr = o_cnt + 256;
-  const size_t scr = generic ? (size_t)std::min<int64_t>(nq, kGenericGrid) *
-                                   generic_scratch_per_block(cl, f.deriv) * 8
+  int64_t longest = 0;  // primitive tuples, screened ones among them
+  for (const int2& v : q) {
+    const PairSet& S = opt ? opt->pairs : local_pairs;
+    longest = std::max<int64_t>(longest, (int64_t)S.np[v.x] * S.np[v.y]);
+  }
+  const size_t scr = generic ? (size_t)generic_scratch(cl, f.deriv, nq, longest) * 8
                              : 0;
   const size_t o_jobs = align256(o_scr + scr);
   const size_t o_sout = o_jobs + align256(jobs.size() * sizeof(SpinorJob));
@@ -1673,7 +1721,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   double* dout = (double*)(A + o_out);
   unsigned long long* dcnt = (unsigned long long*)(A + o_cnt);
   launch_bin_kernels(fam, cl, variant, generic, ks[variant], pd, cutoff,
-                     (const int2*)(A + o_q), nullptr, nq, dout, 0, block, lanes_end,
+                     (const int2*)(A + o_q), nullptr, nq, dout, 0, block, lanes_end, longest,
                      generic ? (double*)(A + o_scr) : nullptr, dcnt, T.stream);
   int d[4] = {n[0], n[1], n[2], n[3]};
   if (dims)
@@ -2183,7 +2231,7 @@ int cintx_plan_execute_graph(cintx_plan* plan, double* out_dev) {
         for (int c = 0; c < kChains - 1; ++c) HIPCHK(hipStreamWaitEvent(C.branch[c], ev[0], 0));
         size_t n_other = 0, n_gen = 0;
         for (size_t i = 0; i < plan->bins.size(); ++i) {
-          const int chain = plan->bins[i].generic ? (int)(n_gen++ % plan->scratch_chains)
+          const int chain = plan->bins[i].runtime_class() ? (int)(n_gen++ % plan->scratch_chains)
                                                   : (int)(n_other++ % kChains);
           plan_launch_bin(plan, i, out, false, chain ? C.branch[chain - 1] : C.stream, chain);
         }
@@ -2399,7 +2447,7 @@ int cintx_plan_bin_stats(const cintx_plan* plan, int64_t nmax, int* cls, int64_t
       if (cls) {
         for (int c = 0; c < 4; ++c) cls[6 * i + c] = b.l[c];
         cls[6 * i + 4] = b.prec;
-        cls[6 * i + 5] = b.generic ? 1 : 0;
+        cls[6 * i + 5] = b.runtime_class() ? 1 : 0;
       }
       if (ntuples) ntuples[i] = (int64_t)b.q.size();
       if (ms) ms[i] = b.last_ms;
@@ -2430,8 +2478,8 @@ int cintx_plan_autotune(cintx_plan* plan, int reps) {
       if (b.generic || b.q.empty()) continue;
       int best = b.variant;
       double best_ms = 1e300;
-      for (int v = 0; v < 2 * kVariants; ++v) {
-        if (!variant_info(plan, b, v).fn) continue;
+      for (int v = 0; v <= kRuntimeClass; ++v) {
+        if (v == kRuntimeClass ? !b.small : !variant_info(plan, b, v).fn) continue;
         b.variant = v;
         auto timed = [&]() {
           HIPCHK(hipEventRecord(e0, C.stream));
@@ -2456,7 +2504,8 @@ int cintx_plan_autotune(cintx_plan* plan, int reps) {
       }
       b.variant = best;
       b.last_ms = best_ms;
-      tuned_slot(plan, b) = (signed char)best;
+      // (the runtime-class kernel wins by the size of this bin: no record)
+      if (best != kRuntimeClass) tuned_slot(plan, b) = (signed char)best;
     }
   });
 }
@@ -2483,12 +2532,13 @@ int cintx_plan_bin_variants(const cintx_plan* plan, int64_t nmax, int* variant, 
       const Bin& b = plan->bins[i];
       int nv = 0;
       for (int v = 0; v < 2 * kVariants; ++v) nv += variant_info(plan, b, v).fn ? 1 : 0;
+      const bool rc = b.runtime_class();
       const KernelInfo& k = variant_info(plan, b, b.variant);
-      if (variant) variant[i] = b.generic ? -1 : b.variant;
-      if (nvariants) nvariants[i] = nv;
-      if (lanes) lanes[i] = b.generic ? 256 : k.lanes_per_tuple;
-      if (prims) prims[i] = b.generic ? 1 : k.prims_per_step;
-      if (tuples_per_block) tuples_per_block[i] = b.generic ? 1 : k.tuples_per_block;
+      if (variant) variant[i] = b.generic ? -1 : rc ? nv : b.variant;
+      if (nvariants) nvariants[i] = nv + (b.small ? 1 : 0);
+      if (lanes) lanes[i] = rc ? 256 : k.lanes_per_tuple;
+      if (prims) prims[i] = rc ? 1 : k.prims_per_step;
+      if (tuples_per_block) tuples_per_block[i] = rc ? 1 : k.tuples_per_block;
     }
   });
 }
@@ -2864,7 +2914,7 @@ static void jk_enqueue(cintx_plan* plan, const double* Dsym, double* dJ, double*
   size_t n_other = 0, n_gen = 0;
   for (size_t i = 0; i < plan->bins.size(); ++i) {
     const Bin& b = plan->bins[i];
-    const int chain = b.generic ? (int)(n_gen++ % std::min(plan->scratch_chains, nchain))
+    const int chain = b.runtime_class() ? (int)(n_gen++ % std::min(plan->scratch_chains, nchain))
                                 : (int)(n_other++ % nchain);
     hipStream_t st = chain ? C.branch[chain - 1] : C.stream;
     if (variant_info_jk(plan, b, b.variant).fn) {
@@ -2872,8 +2922,8 @@ static void jk_enqueue(cintx_plan* plan, const double* Dsym, double* dJ, double*
       continue;
     }
     plan_launch_bin(plan, i, plan->d_out, false, st, chain);
-    HIPCHK(launch_jk_digest(plan->d_out, b.out_base, b.block, b.d_q, (int64_t)b.q.size(),
-                            plan->d_pair_sh, plan->d_ao_off, plan->d_shl_l, Dsym, dJ, dK, nao,
+    HIPCHK(launch_jk_digest(plan->d_out, b.out_base, b.block, b.d_q, b.d_place,
+                            (int64_t)b.q.size(), plan->d_pair_sh, plan->d_ao_off, plan->d_shl_l, Dsym, dJ, dK, nao,
                             st));
   }
   if (ev) {

@@ -265,9 +265,11 @@ int cintx_plan_work(cintx_plan *plan, double *prim_tuples, double *root_evals, d
  * FP64 instantiations (variants 6..11 = FP64 variant 0..5): FP32 without packed
  * math issues at the FP64 rate on CDNA4 and wins only where it saves
  * registers or LDS bytes.  cintx_plan_set_variant forces one variant (0..5)
- * on every bin that has it (variant 0 otherwise); cintx_plan_bin_variants
- * reports per bin: variant in use (-1: runtime-class kernel), variants
- * available, lanes per tuple, primitive tuples per step (for one lane per
+ * on every bin that has it (variant 0 otherwise).  Untuned bins choose by
+ * their size; a small bin may take the runtime-class kernel, which then is
+ * one more variant of that bin, the last.  cintx_plan_bin_variants reports per
+ * bin: variant in use (-1: a class that has only the runtime-class kernel),
+ * variants available, lanes per tuple, primitive tuples per step (for one lane per
  * tuple: row chunks), tuples per workgroup. */
 int cintx_plan_autotune(cintx_plan *plan, int reps);
 int cintx_plan_set_variant(cintx_plan *plan, int variant);

@@ -867,3 +867,38 @@ def test_lanes_shared_by_a_tuple(oracle, count):
         tol = 1e-12 * (1 + np.abs(eri).max()) * np.abs(D).sum()
         assert np.abs(J - Jr).max() <= tol and np.abs(K - Kr).max() <= tol
         p.close()
+
+
+@pytest.mark.parametrize("count", [1, 7, 300])
+def test_small_launches_of_the_runtime_class_kernel(oracle, count):
+    """Classes with compiled kernels whose small launches take the
+    runtime-class kernel, a tuple on several workgroups: one tuple, odd
+    counts, blocks of one and of several row chunks, tuples without a
+    surviving primitive tuple among them, and the nabla_i and Cartesian
+    forms; the same as a graph."""
+    mol = M.config(5)
+    rng = np.random.default_rng(120 + count)
+    ls = mol.bas[:, 1]
+    long = np.nonzero(mol.bas[:, 2] >= 3)[0]
+    by_l = {l: [int(s) for s in long if ls[s] == l] for l in range(5)}
+    pairs = [(2, 2, 2, 2), (2, 2, 2, 1), (4, 4, 1, 0), (3, 1, 2, 2), (4, 2, 3, 1)]
+    tuples = []
+    for cls in pairs:
+        for _ in range(max(1, count // len(pairs))):
+            a = [by_l[l][int(rng.integers(0, 3))] for l in cls]  # near: little is screened
+            tuples.append(tuple(a))
+    far = (by_l[2][0], by_l[2][-1], by_l[2][1], by_l[2][-2])
+    tuples.append(far)
+    p = capi.Plan("int2e_sph", mol.atm, mol.bas, mol.env, tuples)
+    assert any(b["generic"] for b in p.bin_stats())
+    p.execute(graph=True)
+    p.sync()
+    p.fill_output(np.nan)
+    p.execute(graph=True)
+    p.sync()
+    ref, _, _ = oracle_blocks(oracle, "int2e_sph", tuples, mol)
+    assert_parity(p.output(), ref)
+    p.close()
+    check_plan(oracle, "int2e_sph", tuples, mol)
+    check_plan(oracle, "int2e_ip1_sph", tuples[:40], mol)
+    check_plan(oracle, "int2e_cart", tuples[:40], mol)
