@@ -237,7 +237,19 @@ def variants(deriv, prec, ls):
             out.append(c)
     if ne <= 27:  # the register path won every such class by 3-10x
         return out[:2]
-    return out[:6]
+    out = out[:6]
+    if not is_high_l(deriv, ls):
+        # the default among the wide shapes: the i rows, or with many (k, l)
+        # components (or nabla_i) the most lanes with several primitive
+        # tuples in flight.  They lose at most 5% to fewer lanes on large
+        # launches and win up to 3 times on small ones ((d d|p p), 8,462
+        # tuples: 0.57 ms with 64 lanes, 2.04 ms with 16).
+        rows = [c for c in out if c[1] & 256] if nrow < 16 else []
+        many = sorted((c for c in out if c[0] > 1 and 1 < c[1] < 256), key=lambda c: -c[0])
+        for c in (rows or many)[:1]:
+            out.remove(c)
+            out.insert(0, c)
+    return out
 
 
 # Translation units of the larger one-lane variants are compiled with larger
