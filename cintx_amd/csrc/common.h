@@ -19,8 +19,6 @@ namespace cx {
 
 constexpr int kMaxL = 4;          // largest shell l on the hot path (g)
 constexpr int kMaxRoots = 14;     // table covers n = 1 .. kMaxRoots
-constexpr int kRysDeg = 11;       // Chebyshev degree per unit x-interval
-constexpr int kRysNc = kRysDeg + 1;
 constexpr int kC2sL = 6;          // c2s table covers l = 0 .. kC2sL
 constexpr int kC2sM = 2 * kC2sL + 1;
 constexpr int kC2sC = (kC2sL + 1) * (kC2sL + 2) / 2;
@@ -29,10 +27,28 @@ __host__ __device__ constexpr int ncart(int l) { return (l + 1) * (l + 2) / 2; }
 __host__ __device__ constexpr int nsph(int l) { return 2 * l + 1; }
 __host__ __device__ constexpr double rys_largex(int n) { return 35.0 + 5.0 * n; }
 
-// Rys table: for n in 1..kMaxRoots, x in [0, largex(n)) split into unit
-// intervals; per interval, per root r: kRysNc Chebyshev coefficients of
-// s_r = t_r^2 = u_r/(1+u_r) followed (after all n roots) by those of w_r.
+// Rys table: for n in 1..kMaxRoots, per root r, x in [0, largex(n)) split
+// into kRysSub intervals per unit; per interval kRysNc pairs of
+// coefficients, ascending powers of the distance from the middle, of
+// s_r = t_r^2 = u_r/(1+u_r) (or of -q_r, q = 1 - s) and of w_r.
 // For x >= largex(n) the asymptotic rule s = R/x, w = W/sqrt(x) is used.
+//
+// Half-unit intervals with powers up to 10 (one fused multiply-add per
+// coefficient): the relative error of s, q and w is at most 2.4e-16, 2.3e-16
+// and 4.2e-16 for n up to 14, against 3.5e-16, 3.1e-16 and 5.7e-16 of a
+// Chebyshev sum of degree 11 on whole units, which takes two operations per
+// coefficient.  Quarter units with 9 coefficients are as exact and as fast in
+// the plain kernels, but their blocks (52 KB for n = 2 instead of 32 KB, in
+// LDS) cost the fused J/K kernels 4% in occupancy; half units with 10
+// coefficients lose half a digit of w.  11 pairs are an odd number of 16-byte
+// units, so that lanes of different intervals spread over all LDS banks.
+constexpr int kRysSub = 2;
+constexpr int kRysNc = 11;
+__host__ __device__ constexpr int rys_intervals(int n) { return (int)rys_largex(n) * kRysSub; }
+// Doubles of the table block of n roots (roots x intervals x pairs).
+__host__ __device__ constexpr int rys_block_doubles(int n) {
+  return n * rys_intervals(n) * kRysNc * 2;
+}
 struct RysTable {
   const double* coef;   // device
   const double* large;  // device: per n at n(n-1): R[0..n-1], W[0..n-1]

@@ -5,7 +5,7 @@
 //   * a workgroup holds Q shell tuples, T lanes per tuple (T | 64, so a tuple
 //     never straddles a wavefront);
 //   * per primitive tuple: the T lanes evaluate the NR Rys roots from the
-//     Chebyshev table (lane r -> root r), then the 3*NR (axis, root) recurrence
+//     fitted table (lane r -> root r), then the 3*NR (axis, root) recurrence
 //     chains (2D VRR + bra/ket HRR, registers only) and store the 4D g tensor
 //     in LDS as g[axis][i][j][k][l][root], then every lane accumulates its
 //     Cartesian elements sum_r gx*gy*gz in registers;
@@ -46,50 +46,79 @@ __host__ __device__ constexpr void cart_decode(int l, int c, int& lx, int& ly, i
   lx = ly = lz = 0;
 }
 
-// Rys rule for n roots, root r, argument x: s = t^2 = u/(1+u), q = 1 - s and
-// the weight (rys_roots.c:57-123 regimes: Chebyshev table below 35+5n,
+// y = 1/sqrt(v) and r = 1/v of a positive v, each within one unit in the last
+// place: one step of third order from v_rsq_f64 (23 bits), with the rounding
+// of v y carried along.  A division and a square root, with their scaling
+// and fix-up steps, take three times the instructions, which counts where
+// the vector units bound a kernel: they are 58 to 75% busy in the one-lane
+// kernels, and (p s|p s), 1,733,629 tuples, 1.10e8 primitive tuples, took
+// 1.41 ms with both and the Chebyshev sums, 1.23 ms with the table alone
+// changed and takes 1.07 ms.
+__device__ __forceinline__ void rsqrt_rcp(double v, double& y, double& r) {
+  const double y0 = __builtin_amdgcn_rsq(v);
+  const double t = v * y0;
+  const double e = fma(-t, y0, 1.0) - fma(v, y0, -t) * y0;
+  y = fma(y0 * e, fma(e, 0.375, 0.5), y0);
+  r = y * y;
+  r = fma(r, fma(-v, r, 1.0), r);
+}
+
+// What the roots of one argument share: the table's interval and the distance
+// from its middle, or, from largex on, 1/x and 1/sqrt(x).
+struct RysArg {
+  bool far;
+  int iv;
+  double x, t, y;  // the argument; the distance, or 1/x; 1/sqrt(x)
+};
+__device__ __forceinline__ RysArg rys_arg(int n, double x) {
+  RysArg p;
+  p.far = !(x < rys_largex(n));
+  p.x = x;
+  p.y = 0;
+  if (p.far) {
+    p.iv = 0;
+    p.x = x > 1e300 ? 1e300 : x;  // an overflowed x: s and w vanish; NaN stays
+    rsqrt_rcp(p.x, p.y, p.t);
+  } else {
+    p.iv = (int)(x * kRysSub);
+    p.t = x - (p.iv + 0.5) / kRysSub;
+  }
+  return p;
+}
+
+// Rys rule for n roots, root r: s = t^2 = u/(1+u), q = 1 - s and
+// the weight (rys_roots.c:57-123 regimes: fitted table below 35+5n,
 // asymptotic Hermite rule above).  The table holds, per root and interval,
-// the fit of the smaller of s and q; a fitted q is stored negated.
+// the fit of the smaller of s and q; a fitted q is stored negated.  The
+// coefficients of both series of one power lie side by side (one 16-byte read).
 __device__ __forceinline__ void rys_eval_at(const double* __restrict__ cn,
                                             const double* __restrict__ large, int n, int r,
-                                            double x, double& s, double& q, double& w) {
-  if (!(x < rys_largex(n))) {
+                                            const RysArg& p, double& s, double& q, double& w) {
+  if (p.far) {
     const double* L = large + n * (n - 1);
-    s = L[r] / x;
+    const double R = L[r], v = R * p.t;
+    s = fma(p.t, fma(-p.x, v, R), v);  // R / x, correctly rounded but for a few
     q = 1.0 - s;
-    w = L[n + r] / sqrt(x);
+    w = L[n + r] * p.y;
     return;
   }
-  int iv = (int)x;
-  double t = 2.0 * (x - (double)iv) - 1.0;
-  double t2 = t + t;
-  const double* cu = cn + ((size_t)iv * 2 * n + r) * kRysNc;
-  const double* cw = cu + (size_t)n * kRysNc;
-  double bu1 = 0, bu2 = 0, bw1 = 0, bw2 = 0;
+  const double2* c = reinterpret_cast<const double2*>(cn) + (r * rys_intervals(n) + p.iv) * kRysNc;
+  double2 h = c[kRysNc - 1];
 #pragma unroll
-  for (int k = kRysDeg; k >= 1; --k) {
-    double bu0 = fma(t2, bu1, cu[k] - bu2);
-    double bw0 = fma(t2, bw1, cw[k] - bw2);
-    bu2 = bu1;
-    bu1 = bu0;
-    bw2 = bw1;
-    bw1 = bw0;
+  for (int k = kRysNc - 2; k >= 0; --k) {
+    const double2 ck = c[k];
+    h.x = fma(h.x, p.t, ck.x);
+    h.y = fma(h.y, p.t, ck.y);
   }
-  const double v = fma(t, bu1, cu[0] - bu2);
-  const double small = fabs(v);
-  s = v < 0 ? 1.0 - small : small;
-  q = v < 0 ? small : 1.0 - small;
-  w = fma(t, bw1, cw[0] - bw2);
+  const double small = fabs(h.x);
+  s = h.x < 0 ? 1.0 - small : small;
+  q = h.x < 0 ? small : 1.0 - small;
+  w = h.y;
 }
 
 __device__ __forceinline__ void rys_eval(const RysTable& tab, int n, int r, double x, double& s,
                                          double& q, double& w) {
-  rys_eval_at(tab.coef + tab.off[n], tab.large, n, r, x, s, q, w);
-}
-
-// Doubles of the table block of n roots (intervals x 2n series x coefficients).
-__host__ __device__ constexpr int rys_block_doubles(int n) {
-  return (int)rys_largex(n) * 2 * n * kRysNc;
+  rys_eval_at(tab.coef + tab.off[n], tab.large, n, r, rys_arg(n, x), s, q, w);
 }
 
 // Workgroups are dispatched in index order, round-robin over the 8 XCDs, and
@@ -442,12 +471,12 @@ struct ClassShape {
   static constexpr int NFT = (NF + T - 1) / T;                     // T == 1 path
   static constexpr int NSC = 16;  // per-primitive scalars shared in LDS
   // one-lane path, fused J/K: (k, l) output pairs staged per pass for the
-  // 256 lanes of a workgroup within 128 KB of dynamic LDS (the static LDS
-  // of these kernels, the Rys table block, stays below 30 KB)
+  // 256 lanes of a workgroup within 104 KB of dynamic LDS (the static LDS
+  // of these kernels, the Rys table block, stays below 54 KB of the 160 KB)
   // (never more than the (k, l) pairs a chunk reaches, so that small
   // classes keep the occupancy of their plain kernels)
   static constexpr int jk_rows_per_pass() {
-    const int rpp = 64 / (nout(LI) * nout(LJ));
+    const int rpp = 52 / (nout(LI) * nout(LJ));
     const int reach = (LK < 2 && LL < 2) ? RPC : nout(LK) * nout(LL);
     return rpp < 1 ? 1 : (rpp < reach ? rpp : reach);
   }
@@ -570,11 +599,11 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   (void)lds;
   constexpr bool F64 = sizeof(R) == sizeof(double);
   constexpr int NCH = S::NCH, RPC = S::RPC, CE = RPC * NB;  // elements per chunk
-  // up to 3 roots the table block of this n (<= 29 KB) is copied to LDS once
+  // up to 3 roots the table block of this n (<= 53 KB) is copied to LDS once
   // per workgroup: the coefficient reads of every root then hit LDS instead
   // of scattered L2 lines
   constexpr bool LTAB = NR <= 3;
-  __shared__ double stab[LTAB ? rys_block_doubles(NR) : 1];
+  __shared__ __attribute__((aligned(16))) double stab[LTAB ? rys_block_doubles(NR) : 2];
   const double* coefn = a.rys.coef + a.rys.off[NR];
   if constexpr (LTAB) {
     for (int i = threadIdx.x; i < rys_block_doubles(NR); i += blockDim.x) stab[i] = coefn[i];
@@ -682,15 +711,17 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
         p.prb[d] = IBASE ? pr : -wi * rji[d];
         p.qrk[d] = qb[d];
       }
-      p.inv_sum = 1.0 / (p.aij + akl);
+      double root_inv;
+      rsqrt_rcp(p.aij + akl, root_inv, p.inv_sum);
       p.hij = pi[5];
       p.hkl = hkl;
       p.a1 = p.aij * akl;
       p.a0 = p.a1 * p.inv_sum;
       // sqrt(a0/a1^3) = 1/(a1 sqrt(aij+akl)) = 4 hij hkl sqrt(inv_sum)
       const double fac = a.common * pi[4] * kkl;
-      const double fac1 = 4.0 * p.hij * hkl * sqrt(p.inv_sum) * fac;
+      const double fac1 = 4.0 * p.hij * hkl * root_inv * fac;
       const double x = p.a0 * rr;
+      const RysArg ra = rys_arg(NR, x);
       const R ai2 = DERIV ? (R)(-2.0 * pi[7]) : (R)0;
       if (ch == 0) ++nsurv;
       if constexpr (!F64) {
@@ -705,7 +736,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
       if constexpr (ROOTS_FIRST) {
 #pragma unroll
         for (int r = 0; r < NR; ++r)
-          rys_eval_at(coefn, a.rys.large, NR, r, x, rs[r], rq[r], rw[r]);
+          rys_eval_at(coefn, a.rys.large, NR, r, ra, rs[r], rq[r], rw[r]);
       }
 #pragma unroll 1
       for (int r = 0; r < NR; ++r) {
@@ -715,7 +746,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
           qr = rq[r];
           wr = rw[r];
         } else {
-          rys_eval_at(coefn, a.rys.large, NR, r, x, sr, qr, wr);
+          rys_eval_at(coefn, a.rys.large, NR, r, ra, sr, qr, wr);
         }
         const double wz = wr * fac1;
 #pragma unroll
@@ -1007,10 +1038,11 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
             pb[d] = ib ? pr : -pi[1] * rji[d];
             qb[d] = KBASE ? qr : -pk[1] * rlk[d];
           }
-          const double inv_sum = 1.0 / (aij + akl);
+          double root_inv, inv_sum;
+          rsqrt_rcp(aij + akl, root_inv, inv_sum);
           const double hij = pi[5], hkl = pk[5];
           const double fac = a.common * pi[4] * pk[4];
-          const double fac1 = 4.0 * hij * hkl * sqrt(inv_sum) * fac;
+          const double fac1 = 4.0 * hij * hkl * root_inv * fac;
           const double x = aij * akl * inv_sum * rr;
           double sr, qr, w;
           rys_eval(a.rys, NR, r, x, sr, qr, w);
@@ -1270,7 +1302,8 @@ hipError_t launch_class(const EriArgs& a, hipStream_t s) {
   // the one-lane kernels stage their blocks for a fused J/K in dynamic LDS
   size_t dyn = 0;
   if constexpr (S::T == 1 && S::JK) {
-    static_assert(S::jk_lds_bytes() <= 128 * 1024, "fused J/K staging");
+    static_assert(S::jk_lds_bytes() + (S::NR <= 3 ? rys_block_doubles(S::NR) * 8 : 0) <= 160 * 1024,
+                  "fused J/K staging");
     dyn = S::jk_lds_bytes();
   }
   hipLaunchKernelGGL((eri_class_kernel<LI, LJ, LK, LL, DERIV, R, TT, PP>), dim3((unsigned)nblk),

@@ -443,10 +443,11 @@ __global__ void __launch_bounds__(256, gen_waves(DERIV, LEVEL))
               prb[d] = ib ? pr : -pi[1] * rji[d];
               qrk[d] = kb ? qk : -pk[1] * rlk[d];
             }
-            const double inv_sum = 1.0 / (aij + akl);
+            double root_inv, inv_sum;
+            rsqrt_rcp(aij + akl, root_inv, inv_sum);
             const double hij = pi[5], hkl = pk[5];
             const double fac = a.common * pi[4] * pk[4];
-            const double fac1 = 4.0 * hij * hkl * sqrt(inv_sum) * fac;
+            const double fac1 = 4.0 * hij * hkl * root_inv * fac;
             const double a0 = aij * akl * inv_sum;
             const double x = a0 * rr;
             double sr, qr, w;

@@ -2728,8 +2728,8 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
   });
 }
 
-// Rys rule from the Chebyshev table, evaluated on the host (same table and
-// Clenshaw recurrence as rys_eval in eri_device.h).
+// Rys rule from the table, evaluated on the host (same table and Horner
+// scheme as rys_eval in eri_device.h).
 int cintx_rys_eval_host(int n, const double* x, int64_t nx, double* u, double* w) {
   return guarded([&] {
     if (n < 1 || n > kMaxRoots) fail(CINTX_STATUS_INVALID_INPUT, "nroots out of range");
@@ -2751,24 +2751,19 @@ int cintx_rys_eval_host(int n, const double* x, int64_t nx, double* u, double* w
           w[i * n + r] = L[n + r] / std::sqrt(xi);
           continue;
         }
-        int iv = (int)xi;
-        double t = 2.0 * (xi - iv) - 1.0, t2 = t + t;
-        const double* cu = coef.data() + off[n] + ((size_t)iv * 2 * n + r) * kRysNc;
-        const double* cw = cu + (size_t)n * kRysNc;
-        double bu1 = 0, bu2 = 0, bw1 = 0, bw2 = 0;
-        for (int k = kRysDeg; k >= 1; --k) {
-          double bu0 = std::fma(t2, bu1, cu[k] - bu2);
-          double bw0 = std::fma(t2, bw1, cw[k] - bw2);
-          bu2 = bu1;
-          bu1 = bu0;
-          bw2 = bw1;
-          bw1 = bw0;
+        constexpr int nc = kRysNc;
+        const int iv = (int)(xi * kRysSub);
+        const double t = xi - (iv + 0.5) / kRysSub;
+        const double* c = coef.data() + off[n] + ((size_t)r * rys_intervals(n) + iv) * nc * 2;
+        double v = c[2 * nc - 2], wr = c[2 * nc - 1];
+        for (int k = nc - 2; k >= 0; --k) {
+          v = std::fma(v, t, c[2 * k]);
+          wr = std::fma(wr, t, c[2 * k + 1]);
         }
-        double v = std::fma(t, bu1, cu[0] - bu2);
         double small = std::fabs(v);
         double sr = v < 0 ? 1.0 - small : small, qr = v < 0 ? small : 1.0 - small;
         u[i * n + r] = sr / qr;
-        w[i * n + r] = std::fma(t, bw1, cw[0] - bw2);
+        w[i * n + r] = wr;
       }
     }
   });

@@ -2,7 +2,7 @@
 // (log x, nroots) to initial roots and weights, trained on the device by the
 // kernels below (forward + backward + Adam, FP32), followed by FP64 Newton
 // steps on the moment equations sum_i w_i s_i^m = F_m(x), m = 0..2n-1.  The
-// Chebyshev-table rule (the plain solver) judges the polished rule: where any
+// fitted-table rule (the plain solver) judges the polished rule: where any
 // root u_i or weight w_i differs from it by more than 1e-14 relative, the
 // table rule is returned instead.
 //

@@ -7,9 +7,9 @@
 // table node in 80-bit long double by discretising the measure with
 // Gauss-Legendre nodes and running the Stieltjes procedure (W. Gautschi,
 // SIAM J. Sci. Stat. Comput. 3 (1982) 289) followed by the Golub-Welsch
-// eigen-solve (implicit QL).  The device evaluates degree-11 Chebyshev fits
+// eigen-solve (implicit QL).  The device evaluates polynomial fits
 // of s_r(x) = t_r^2 = u_r/(1+u_r) (or of q_r = 1 - s_r where s_r > 1/2, stored
-// negated) and w_r(x) on unit x-intervals below 35+5n (the LARGEX bound of
+// negated) and w_r(x) on short x-intervals below 35+5n (the LARGEX bound of
 // rys_roots.c:67) and the asymptotic Hermite rule s = R/x, w = W/sqrt(x)
 // above it.  Keeping s and q rather than u makes every per-root coefficient
 // of the recurrences division-free without losing accuracy near s = 1.
@@ -27,6 +27,7 @@ namespace cx {
 namespace {
 
 constexpr int kGlMax = 256;
+constexpr int kFit = 12;  // nodes of the fit of one unit of x
 
 struct GaussLegendre {
   long double t[kGlMax], w[kGlMax];
@@ -192,45 +193,83 @@ void rys_table_build(std::vector<double>& coef, std::vector<double>& large,
   off[0] = 0;
   for (int n = 1; n <= kMaxRoots; ++n) {
     off[n] = (int)total;
-    int nint = (int)rys_largex(n);
-    total += (size_t)nint * 2 * n * kRysNc;
+    total += rys_block_doubles(n);
   }
   coef.assign(total, 0.0);
   large.assign((size_t)kMaxRoots * (kMaxRoots + 1), 0.0);
   const long double pi = 3.14159265358979323846264338327950288L;
   for (int n = 1; n <= kMaxRoots; ++n) {
-    int nint = (int)rys_largex(n);
+    const int nint = (int)rys_largex(n), sub = kRysSub, nc = kRysNc;
+    // cos(pi j (k + 1/2) / m): the values of T_j at the m nodes
+    long double at_fit[kFit][kFit], at_nc[kFit][kFit];
+    for (int k = 0; k < kFit; ++k)
+      for (int j = 0; j < kFit; ++j) {
+        at_fit[k][j] = cosl(pi * j * (k + 0.5L) / kFit);
+        at_nc[k][j] = cosl(pi * j * (k + 0.5L) / nc);
+      }
 #pragma omp parallel for schedule(dynamic, 1)
     for (int iv = 0; iv < nint; ++iv) {
-      long double su[kRysNc][kMaxRoots], sw[kRysNc][kMaxRoots];
-      for (int k = 0; k < kRysNc; ++k) {
-        long double tk = cosl(pi * (k + 0.5L) / kRysNc);
-        long double x = iv + 0.5L * (tk + 1.0L);
+      long double val[kFit][2 * kMaxRoots];  // s of every root, then w
+      for (int k = 0; k < kFit; ++k) {
         long double s[kMaxRoots + 2], w[kMaxRoots + 2];
-        rys_rule_ld(n, x, s, w);
+        rys_rule_ld(n, iv + 0.5L * (at_fit[k][1] + 1.0L), s, w);
         for (int r = 0; r < n; ++r) {
-          su[k][r] = s[r];  // t^2; u = s/(1-s) is formed only where needed
-          sw[k][r] = w[r];
+          val[k][r] = s[r];  // t^2; u = s/(1-s) is formed only where needed
+          val[k][n + r] = w[r];
         }
       }
-      double* blk = coef.data() + off[n] + (size_t)iv * 2 * n * kRysNc;
-      for (int r = 0; r < n; ++r) {
-        // Fit whichever of s and q = 1-s is the smaller on this interval, so
+      for (int f = 0; f < 2 * n; ++f) {
+        const int r = f < n ? f : f - n;
+        // Fit whichever of s and q = 1-s is the smaller on this unit, so
         // both come out with full relative accuracy (q matters near s = 1);
         // a fitted q is stored negated, which the evaluator detects by sign.
-        long double smid = 0;
-        for (int k = 0; k < kRysNc; ++k) smid += su[k][r];
-        const bool fit_q = smid / kRysNc > 0.5L;
-        for (int j = 0; j < kRysNc; ++j) {
-          long double cu = 0, cw = 0;
-          for (int k = 0; k < kRysNc; ++k) {
-            long double tj = cosl(pi * j * (k + 0.5L) / kRysNc);
-            cu += (fit_q ? -(1.0L - su[k][r]) : su[k][r]) * tj;
-            cw += sw[k][r] * tj;
+        if (f < n) {
+          long double smid = 0;
+          for (int k = 0; k < kFit; ++k) smid += val[k][f];
+          if (smid / kFit > 0.5L)
+            for (int k = 0; k < kFit; ++k) val[k][f] = -(1.0L - val[k][f]);
+        }
+        long double cheb[kFit];
+        for (int j = 0; j < kFit; ++j) {
+          cheb[j] = 0;
+          for (int k = 0; k < kFit; ++k) cheb[j] += val[k][f] * at_fit[k][j];
+          cheb[j] *= (j == 0 ? 1.0L : 2.0L) / kFit;
+        }
+        // the fit of the unit, fitted again on each of its intervals with
+        // fewer terms and expanded in powers of the distance from the middle
+        for (int h = 0; h < sub; ++h) {
+          const long double half = 0.5L / sub, mid = (h + 0.5L) / sub;
+          long double at[kFit];
+          for (int k = 0; k < nc; ++k) {
+            const long double t = 2.0L * (mid + half * at_nc[k][1]) - 1.0L;
+            long double b1 = 0, b2 = 0;
+            for (int j = kFit - 1; j >= 1; --j) {
+              const long double b = 2.0L * t * b1 - b2 + cheb[j];
+              b2 = b1;
+              b1 = b;
+            }
+            at[k] = t * b1 - b2 + cheb[0];
           }
-          long double sc = (j == 0 ? 1.0L : 2.0L) / kRysNc;
-          blk[(size_t)r * kRysNc + j] = (double)(cu * sc);
-          blk[(size_t)(n + r) * kRysNc + j] = (double)(cw * sc);
+          long double pw[kFit] = {0}, t0[kFit] = {0}, t1[kFit] = {0};
+          t0[0] = 1;
+          t1[1] = 1;
+          for (int j = 0; j < nc; ++j) {  // t0 = T_j, t1 = T_(j+1) by powers
+            long double c = 0;
+            for (int k = 0; k < nc; ++k) c += at[k] * at_nc[k][j];
+            c *= (j == 0 ? 1.0L : 2.0L) / nc;
+            for (int i = 0; i < nc; ++i) pw[i] += c * t0[i];
+            for (int i = nc - 1; i >= 0; --i) {
+              const long double t2 = (i > 0 ? 2.0L * t1[i - 1] : 0.0L) - t0[i];
+              t0[i] = t1[i];
+              t1[i] = t2;
+            }
+          }
+          double* blk = coef.data() + off[n] + ((size_t)r * nint * sub + iv * sub + h) * nc * 2;
+          long double scale = 1;
+          for (int i = 0; i < nc; ++i) {
+            blk[2 * i + (f < n ? 0 : 1)] = (double)(pw[i] * scale);
+            scale /= half;
+          }
         }
       }
     }

@@ -82,6 +82,47 @@ def test_device_rys_rule_matches_oracle(oracle):
             assert np.max(np.abs(w[k] - wo) / wo) < tol
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 9, 14])
+def test_device_rys_rule_at_interval_edges(n):
+    """The device rule where its table changes interval and where the
+    asymptotic rule takes over, by the moments sum_r w_r s_r^m = F_m(x)
+    (mpmath, 40 digits).  Tolerance: s and w within two units in the last
+    place and u = s/(1-s) one more, so (m + 2) 5e-16 of the moment.  Past
+    1e300 s and w vanish."""
+    import mpmath as mp
+    mp.mp.dps = 40
+    top = 35.0 + 5 * n
+    edges = np.array([0.5, 1.0, 7.5, 20.0, top - 0.5, top])
+    xs = np.concatenate([[0.0, 1e-300, 0.25], np.nextafter(edges, 0), edges,
+                         np.nextafter(edges, 1e3), [0.75 * top, top + 0.5, 1e300, 1e308, np.inf]])
+    L = capi.lib()
+    L.cintx_rys_eval_device.argtypes = [ctypes.c_int, capi.DP, ctypes.c_int64, capi.DP, capi.DP]
+    u = np.zeros(len(xs) * n)
+    w = np.zeros(len(xs) * n)
+    assert L.cintx_rys_eval_device(n, capi._dp(xs), len(xs), capi._dp(u), capi._dp(w)) == 0
+    u, w = u.reshape(-1, n), w.reshape(-1, n)
+    for k, x in enumerate(xs):
+        if x >= 1e300:
+            assert np.all((u[k] >= 0) & (u[k] < 1e-297) & (w[k] >= 0) & (w[k] < 1e-149)), x
+            continue
+        if x >= top:  # the asymptotic rule itself is good to 1e-13
+            continue
+        s = [mp.mpf(v) / (1 + mp.mpf(v)) for v in u[k]]
+        for m in range(2 * n):
+            a, y = m + mp.mpf(1) / 2, mp.mpf(x)
+            ref = 1 / (2 * a) if x < 1e-200 else mp.gammainc(a, 0, y) / (2 * y ** a)
+            got = mp.fsum(mp.mpf(float(w[k][r])) * s[r] ** m for r in range(n))
+            assert abs(got / ref - 1) < 5e-16 * (m + 2), (x, m)
+    far = xs[(xs >= top) & (xs < 1e300)]
+    uh = np.zeros(len(far) * n)
+    wh = np.zeros(len(far) * n)
+    L.cintx_rys_eval_host.argtypes = [ctypes.c_int, capi.DP, ctypes.c_int64, capi.DP, capi.DP]
+    assert L.cintx_rys_eval_host(n, capi._dp(far), len(far), capi._dp(uh), capi._dp(wh)) == 0
+    sel = (xs >= top) & (xs < 1e300)
+    assert np.allclose(u[sel].ravel(), uh, rtol=1e-15, atol=0)
+    assert np.allclose(w[sel].ravel(), wh, rtol=1e-15, atol=0)
+
+
 def test_int2e_sph_cfg1_full_tensor(oracle):
     mol = M.config(1)
     n = mol.nbas
