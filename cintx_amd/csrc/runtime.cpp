@@ -2087,10 +2087,61 @@ static std::vector<double> abs_coef_env(const int* atm, const int* bas, int nbas
   return eabs;
 }
 
+// How much larger the terms that the transfer of a shell pair sums are than
+// the pair itself.  The FP32 kernels build (x - R_b)^n up to n = l_b + l_o on
+// the centre b of the larger l and transfer l_o of them to the other centre,
+// (x - R_o)^m = sum_k C(m,k) (x - R_b)^k (R_b - R_o)^(m-k): where the product
+// centre P lies near o (a tight shell there, a diffuse one on b) terms of
+// size (|P - R_b| + s + R)^m leave one of size max(|P - R_o|, s)^m, with s =
+// sqrt(1/2p) the width of the product.  Averaged over the primitive pairs
+// with the size of their charge distributions as weights (|c c| exp(-e)
+// p^(-3/2) of charge, its self-repulsion as sqrt(p), and the monomials); equal
+// l: the worse of the two bases, since the tuple's orientation decides.
+static double transfer_growth(const int* atm, const int* bas, const double* env, int sa, int sb) {
+  const int* A = bas + 8 * (size_t)sa;
+  const int* B = bas + 8 * (size_t)sb;
+  const int la = A[1], lb = B[1];
+  if (la == 0 || lb == 0) return 1.0;
+  const double *ra = env + atm[6 * A[0] + 1], *rb = env + atm[6 * B[0] + 1];
+  double rr = 0;
+  for (int d = 0; d < 3; ++d) rr += (ra[d] - rb[d]) * (ra[d] - rb[d]);
+  const double R = std::sqrt(rr);
+  double worst = 1.0;
+  for (int ca = 0; ca < A[3]; ++ca)
+    for (int cb = 0; cb < B[3]; ++cb) {
+      double size = 0, terms = 0;
+      for (int i = 0; i < A[2]; ++i)
+        for (int j = 0; j < B[2]; ++j) {
+          const double ea = env[A[5] + i], eb = env[B[5] + j], p = ea + eb, s = std::sqrt(0.5 / p);
+          const double pa = eb / p * R, pb = ea / p * R;  // |P - R_a|, |P - R_b|
+          const double ga = std::pow((pb + s + R) / std::max(pa, s), la);  // transfer to a
+          const double gb = std::pow((pa + s + R) / std::max(pb, s), lb);
+          const double w = std::fabs(env[A[6] + ca * A[2] + i] * env[B[6] + cb * B[2] + j]) *
+                           std::exp(-ea * eb / p * rr) * std::pow(p, -1.25) *
+                           std::pow(std::max(pa, s), la) * std::pow(std::max(pb, s), lb);
+          size += w;
+          terms += w * (la > lb ? gb : lb > la ? ga : std::max(ga, gb));
+        }
+      if (size > 0) worst = std::max(worst, terms / size);
+    }
+  return worst;
+}
+
+// Whether a tuple of Schwarz bound b (over the absolute coefficients) whose
+// pairs' transfers grow by ga and gb takes the FP32 recurrences: their error
+// stays within a tenth of mixed_threshold.  An FP32 rounding of the terms is
+// 2^-24 ga gb b; over 16,000 uncontracted s, p, d quartets (exponents 0.08 to
+// 5000, 2 to 9 bohr) the error is at most 0.56 of it where it is above 1e-3
+// b, and at most 1e-5 b plus 0.8 of it below.  ((d d|d d) reaches 220 b.)
+static bool fp32_fits(double b, double ga, double gb, double thr) {
+  return b * std::max(1.0, 10.0 * 0x1p-24 * ga * gb) < thr;
+}
+
 // Precision of each tuple of an explicit int2e_sph / int3c2e_sph list in a
 // mixed plan: FP32 recurrences when the Schwarz bound over the absolute
 // coefficients, sqrt((ij|ij)) sqrt((kl|kl)) or sqrt((ij|ij)) sqrt((P|P)),
-// is below mixed_threshold.
+// is below mixed_threshold by as much as the transfers' terms are larger
+// (fp32_fits).
 static std::vector<uint8_t> mixed_selection(int family, const int* atm, int natm,
                                             const int* bas, int nbas, const double* env,
                                             const int* tuples, int64_t nt, double thr) {
@@ -2125,11 +2176,14 @@ static std::vector<uint8_t> mixed_selection(int family, const int* atm, int natm
   }
   const std::vector<double> qp = diag_schwarz(0, atm, natm, bas, nbas, eabs.data(), dpair);
   const std::vector<double> qa = diag_schwarz(4, atm, natm, bas, nbas, eabs.data(), daux);
+  std::vector<double> growth(qp.size());
+  for (size_t k = 0; k < growth.size(); ++k)
+    growth[k] = transfer_growth(atm, bas, env, dpair[4 * k], dpair[4 * k + 1]);
   std::vector<uint8_t> prec((size_t)nt);
   for (int64_t t = 0; t < nt; ++t) {
-    const double b = qp[(size_t)ref[(size_t)t].x] *
-                     (family == 0 ? qp[(size_t)ref[(size_t)t].y] : qa[(size_t)ref[(size_t)t].y]);
-    prec[(size_t)t] = b < thr ? 1 : 0;
+    const size_t x = (size_t)ref[(size_t)t].x, y = (size_t)ref[(size_t)t].y;
+    prec[(size_t)t] = fp32_fits(qp[x] * (family == 0 ? qp[y] : qa[y]), growth[x],
+                                family == 0 ? growth[y] : 1.0, thr);
   }
   return prec;
 }
@@ -2691,8 +2745,13 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
       if (precision == CINTX_PREC_MIXED) {
         // split by bound: FP32 bins for tuples below mixed_threshold
         std::vector<int> lo, hi;
-        std::unordered_map<uint64_t, double> qof;
-        for (const SP& s : sp) qof[((uint64_t)s.a << 32) | (uint32_t)s.b] = qabs[(size_t)s.id];
+        struct PairSize {
+          double q, growth;
+        };
+        std::unordered_map<uint64_t, PairSize> qof;
+        for (const SP& s : sp)
+          qof[((uint64_t)s.a << 32) | (uint32_t)s.b] = {
+              qabs[(size_t)s.id], transfer_growth(atm, bas, env, s.a, s.b)};
         // FP32 without packed math issues at the FP64 rate on CDNA4: the FP32
         // recurrences pay only in classes that must share g through LDS (half
         // the LDS bytes and registers), which are those not placed by work
@@ -2707,9 +2766,13 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
                  !ctx().reg->by_work[0][0][la][lb][lc][ld];
         };
         for (int64_t t = 0; t < nt; ++t) {
-          double b = qof[((uint64_t)tuples[4 * t] << 32) | (uint32_t)tuples[4 * t + 1]] *
-                     qof[((uint64_t)tuples[4 * t + 2] << 32) | (uint32_t)tuples[4 * t + 3]];
-          auto& dst = (b < mixed_threshold && fp32_pays(&tuples[4 * t])) ? lo : hi;
+          const PairSize& x = qof[((uint64_t)tuples[4 * t] << 32) | (uint32_t)tuples[4 * t + 1]];
+          const PairSize& y =
+              qof[((uint64_t)tuples[4 * t + 2] << 32) | (uint32_t)tuples[4 * t + 3]];
+          auto& dst = (fp32_fits(x.q * y.q, x.growth, y.growth, mixed_threshold) &&
+                       fp32_pays(&tuples[4 * t]))
+                          ? lo
+                          : hi;
           dst.insert(dst.end(), tuples.begin() + 4 * t, tuples.begin() + 4 * t + 4);
         }
         plan_add_tuples(P, hi.data(), (int64_t)hi.size() / 4, 0);

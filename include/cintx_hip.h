@@ -192,7 +192,10 @@ size_t cintrs_copy_last_error_message(char *out, size_t out_len);
 
 /* precision modes: FP64 everywhere, or the mixed mode (FP32 recurrences and
  * primitive sums for tuples whose Schwarz bound is below the plan's
- * mixed_threshold, FP64 for the rest and for roots/weights/accumulation). */
+ * mixed_threshold, FP64 for the rest and for roots/weights/accumulation).
+ * An FP32 tuple's error stays within a tenth of mixed_threshold: a pair of a
+ * tight and a distant diffuse shell with l > 0 on both, whose recurrences sum
+ * terms far larger than their result, counts with the size of those terms. */
 #define CINTX_PREC_FP64 0
 #define CINTX_PREC_MIXED 1
 

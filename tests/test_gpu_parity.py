@@ -824,6 +824,57 @@ def test_int3c2e_mixed_cfg4(oracle):
     p.close()
 
 
+@pytest.mark.parametrize("kind", ["tight_diffuse_d", "contracted", "screened", "int3c2e"])
+def test_mixed_plan_error_of_distant_pairs(oracle, kind):
+    """Pairs of a tight and a distant diffuse shell, whose transfer cancels in
+    FP32 (the error of a (d d|d d) quartet was up to 220 times its Schwarz
+    bound): what a mixed plan puts in FP32 stays within a tenth of its
+    threshold (1e-3 here, where an error of the order of the bound shows)."""
+    rng = np.random.default_rng({"tight_diffuse_d": 1, "contracted": 2, "screened": 3,
+                                 "int3c2e": 4}[kind])
+    thr, nfp32, worst = 1e-3, 0, 0.0
+    for _ in range(3):
+        mol = M.Molecule()
+        r = float(rng.uniform(3.0, 7.0))
+        for x in (0.0, r):
+            for _ in range(2):
+                mol.add_atom(1, [x + 0.4 * rng.normal(), 0.4 * rng.normal(), 0.4 * rng.normal()])
+        for a in range(4):
+            for l in range(3):
+                if kind == "tight_diffuse_d":
+                    for lo, hi in ((200.0, 5000.0), (0.1, 1.5)):
+                        e = float(np.exp(rng.uniform(np.log(lo), np.log(hi))))
+                        mol.add_shell(a, l, [e], [[M.gto_norm(l, e)]])
+                else:
+                    n = int(rng.integers(1, 5))
+                    e = np.sort(np.exp(rng.uniform(np.log(0.1), np.log(5000.0), n)))[::-1]
+                    mol.add_shell(a, l, e, [[rng.normal() * M.gto_norm(l, v) for v in e]])
+        mol.build()
+        name = "int3c2e_sph" if kind == "int3c2e" else "int2e_sph"
+        arity = 3 if kind == "int3c2e" else 4
+        if kind == "screened":
+            p = capi.Plan(name, mol.atm, mol.bas, mol.env, screened=(1e-9, 1),
+                          precision=capi.PREC_MIXED, mixed_threshold=thr)
+        else:
+            ls = mol.bas[:, 1]
+            d = np.nonzero(ls == 2)[0] if kind == "tight_diffuse_d" else np.nonzero(ls >= 1)[0]
+            tuples = [tuple(int(s) for s in rng.choice(d, arity)) for _ in range(1500)]
+            p = capi.Plan(name, mol.atm, mol.bas, mol.env, tuples, precision=capi.PREC_MIXED,
+                          mixed_threshold=thr)
+        p.execute()
+        p.sync()
+        got = p.output()
+        t, _ = p.tuples()
+        ref, _, _ = oracle.eval_list(name, [tuple(int(v) for v in q[:arity]) for q in t], mol.atm,
+                                     mol.bas, mol.env, ext=True)
+        nfp32 += p.ntuples_fp32
+        worst = max(worst, float(np.abs(got - ref).max()))
+        p.close()
+    say(f"  {kind}: {nfp32} tuples in FP32, max abs err {worst:.3e}")
+    assert nfp32 > 0
+    assert worst <= thr / 10
+
+
 def test_autotune_keeps_results(oracle):
     mol = M.config(1)
     n = mol.nbas
