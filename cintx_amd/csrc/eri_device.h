@@ -548,7 +548,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   const int64_t q = REG ? (int64_t)sb.first + slot : (int64_t)heavy_first_block() * Q + slot;
   const bool active = q < (REG ? (int64_t)sb.end : a.nq);
   const int2 pq = a.quartets[active ? q : 0];
-  const int64_t place = a.place && active ? a.place[q] : q;  // block of the output
+  const int64_t place = REG && a.place && active ? a.place[q] : q;  // block of the output
   const int boff = a.pair_off[pq.x];
   const int koff = a.pair_off[pq.y];
   const double* gb = a.pair_geo + 8 * (size_t)pq.x;

@@ -13,7 +13,7 @@ namespace cx {
 // The digestion of quartet t by `nl` cooperating lanes (lane index `ln`).
 __device__ __forceinline__ void jk_digest_one(
     const double* __restrict__ eri, int64_t out_base, int64_t block, const int2* __restrict__ q,
-    const int* __restrict__ place, int64_t t, int ln, int nl, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
+    int64_t t, int ln, int nl, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
     const int* __restrict__ shl_l, const double* __restrict__ D, double* __restrict__ J,
     double* __restrict__ K, int nao, bool skip_bra_j = false) {
   const int2 pq = q[t];
@@ -21,24 +21,24 @@ __device__ __forceinline__ void jk_digest_one(
   const int ns[4] = {2 * shl_l[sh[0]] + 1, 2 * shl_l[sh[1]] + 1, 2 * shl_l[sh[2]] + 1,
                      2 * shl_l[sh[3]] + 1};
   const int off[4] = {ao_off[sh[0]], ao_off[sh[1]], ao_off[sh[2]], ao_off[sh[3]]};
-  jk_digest_block(eri + out_base + (place ? place[t] : t) * block, ns, sh, off, ln, nl, D, J, K, nao, skip_bra_j);
+  jk_digest_block(eri + out_base + t * block, ns, sh, off, ln, nl, D, J, K, nao, skip_bra_j);
 }
 
 // Large blocks: one 64-lane workgroup per quartet.
 __global__ void __launch_bounds__(64) jk_digest_kernel(
     const double* __restrict__ eri, int64_t out_base, int64_t block, const int2* __restrict__ q,
-    const int* __restrict__ place, int64_t nq, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
+    int64_t nq, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
     const int* __restrict__ shl_l, const double* __restrict__ D, double* __restrict__ J,
     double* __restrict__ K, int nao) {
   for (int64_t t = blockIdx.x; t < nq; t += gridDim.x)
-    jk_digest_one(eri, out_base, block, q, place, t, threadIdx.x, blockDim.x, pair_sh, ao_off, shl_l, D,
+    jk_digest_one(eri, out_base, block, q, t, threadIdx.x, blockDim.x, pair_sh, ao_off, shl_l, D,
                   J, K, nao);
 }
 
 // Small blocks: one lane per quartet.
 __global__ void __launch_bounds__(256) jk_digest_lane_kernel(
     const double* __restrict__ eri, int64_t out_base, int64_t block, const int2* __restrict__ q,
-    const int* __restrict__ place, int64_t nq, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
+    int64_t nq, const int2* __restrict__ pair_sh, const int* __restrict__ ao_off,
     const int* __restrict__ shl_l, const double* __restrict__ D, double* __restrict__ J,
     double* __restrict__ K, int nao) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256) jk_digest_lane_kernel(
   const int bra0 = __shfl(bra, 0);
   const bool shared = __all(!live || bra == bra0) && bra0 >= 0;
   if (live)
-    jk_digest_one(eri, out_base, block, q, place, t, 0, 1, pair_sh, ao_off, shl_l, D, J, K, nao, shared);
+    jk_digest_one(eri, out_base, block, q, t, 0, 1, pair_sh, ao_off, shl_l, D, J, K, nao, shared);
   if (shared) {
     const int si = pair_sh[bra0].x, sj = pair_sh[bra0].y;
     const int ni = 2 * shl_l[si] + 1, nj = 2 * shl_l[sj] + 1;
@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(256) jk_digest_lane_kernel(
       ok = ao_off[sk];
       ol = ao_off[sl];
       wgt = 2.0 * jk_weight(si, sj, sk, sl);
-      blk = eri + out_base + (place ? place[t] : t) * block;
+      blk = eri + out_base + t * block;
     }
     const int st2 = ni * nj, st3 = ni * nj * nk;
     for (int o = 0; o < ni * nj; ++o) {  // uniform over the wavefront
@@ -85,17 +85,17 @@ __global__ void __launch_bounds__(256) jk_digest_lane_kernel(
 }
 
 hipError_t launch_jk_digest(const double* eri, int64_t out_base, int64_t block, const int2* q,
-                            const int* place, int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
+                            int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
                             const double* D, double* J, double* K, int nao, hipStream_t s) {
   if (nq <= 0) return hipSuccess;
   if (block <= 45) {  // up to (d p|p s): a lane per quartet
     const int64_t grid = (nq + 255) / 256;
     hipLaunchKernelGGL(jk_digest_lane_kernel, dim3((unsigned)grid), dim3(256), 0, s, eri,
-                       out_base, block, q, place, nq, pair_sh, ao_off, shl_l, D, J, K, nao);
+                       out_base, block, q, nq, pair_sh, ao_off, shl_l, D, J, K, nao);
   } else {
     const int grid = (int)std::min<int64_t>(nq, 65536);
     hipLaunchKernelGGL(jk_digest_kernel, dim3(grid), dim3(64), 0, s, eri, out_base, block, q,
-                       place, nq, pair_sh, ao_off, shl_l, D, J, K, nao);
+                       nq, pair_sh, ao_off, shl_l, D, J, K, nao);
   }
   return hipGetLastError();
 }

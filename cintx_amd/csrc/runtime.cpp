@@ -49,7 +49,7 @@ hipError_t launch_jk_sym_copy(const double* src, double* dst, int n, hipStream_t
 hipError_t jk_scratch_address(double** ptr);
 size_t jk_scratch_bytes();
 hipError_t launch_jk_digest(const double* eri, int64_t out_base, int64_t block, const int2* q,
-                            const int* place, int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
+                            int64_t nq, const int2* pair_sh, const int* ao_off, const int* shl_l,
                             const double* D, double* J, double* K, int nao, hipStream_t s);
 hipError_t launch_spinor(const SpinorJob* jobs, int64_t njobs, const double* cart, double* out,
                          const double* tab, const double* c2s, double* scratch, int64_t slice,
@@ -568,12 +568,15 @@ struct Bin {
   std::vector<int2> q;
   int64_t out_base = 0;  // element offset of the bin's first block
   int64_t block = 0;     // elements per block (NS * ncomp)
-  // one-lane launches: tuples before lanes_end[k] that take at most 2^k lanes
-  std::array<int64_t, kSplits> lanes_end{};
-  // block number of every tuple of q, where that is not its own number
+  // one-lane launches: their order of the tuples and the block of each, where
+  // that is not the order of q, and the tuples before lanes_end[k], which take
+  // at most 2^k lanes
+  std::vector<int2> lane_q;
   std::vector<int> place;
+  std::array<int64_t, kSplits> lanes_end{};
   // device pointers (inside the plan blob)
   int2* d_q = nullptr;
+  int2* d_lane_q = nullptr;
   int* d_place = nullptr;
 };
 
@@ -860,15 +863,16 @@ static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);
 static const KernelInfo& variant_info(const cintx_plan* P, const Bin& b, int v);
 static int bin_form(const cintx_plan* P, const Bin& b);
 
-// A bin's blocks are placed by (bra, ket) primitive-pair counts (counting
-// sort), or for the classes of Registry::by_work by surviving primitive
-// tuples (stable).  Its tuples are listed in that order, except that a class
-// with a one-lane kernel always lists them by surviving primitive tuples, so
-// that the lanes of a wavefront, which each walk their own survivors, run
-// equal numbers of iterations and neighbouring tuples take equal numbers of
-// lanes; `place` then holds the block of every tuple.  (The wide kernels'
-// tuples share a workgroup best with equal loop counts, which either order
-// gives them.)
+// A bin's blocks are placed, and its tuples listed, by (bra, ket)
+// primitive-pair counts (counting sort), or for the classes of
+// Registry::by_work by surviving primitive tuples (stable).  A class with a
+// one-lane kernel that is not one of those has a second list for it, by
+// surviving primitive tuples: the lanes of a wavefront, which each walk their
+// own survivors, then run equal numbers of iterations and neighbouring tuples
+// take equal numbers of lanes.  (The wide kernels' workgroups loop to the
+// largest counts among their tuples, and on that list, where equal numbers of
+// survivors come of different counts, nabla_i (p p|p p) of 4 to 541 tuples
+// took up to 1.5 times as long as on the other.)
 static void plan_sort_bins(cintx_plan* P) {
   const PairSet& S = P->pairs;
   const FamilyInfo& f = kFam[P->family];
@@ -889,7 +893,7 @@ static void plan_sort_bins(cintx_plan* P) {
     };
     std::vector<int> key((size_t)n);
     std::vector<int64_t>& pos = remap[bi];  // blocks
-    std::vector<int64_t> by_work;           // places in the list, where not the blocks
+    std::vector<int64_t> by_work;           // places in the one-lane list, where another
     const bool placed_by_work =
         ctx().reg->by_work[f.deriv][bin_form(P, b)][b.l[0]][b.l[1]][b.l[2]][b.l[3]];
     bool one_lane = false;
@@ -934,15 +938,18 @@ static void plan_sort_bins(cintx_plan* P) {
     }
     b.variant = std::max(b.variant, 0);
     b.small = b.variant == kRuntimeClass;
-    const std::vector<int64_t>& at = by_work.empty() ? pos : by_work;
-    std::vector<int2> sorted((size_t)n);
-    for (int64_t i = 0; i < n; ++i) sorted[(size_t)at[(size_t)i]] = b.q[(size_t)i];
-    b.q.swap(sorted);
     if (!by_work.empty()) {
       if (n > INT32_MAX) fail(CINTX_STATUS_MEMORY_LIMIT_EXCEEDED, "too many tuples of one class");
+      b.lane_q.resize((size_t)n);
       b.place.resize((size_t)n);
-      for (int64_t i = 0; i < n; ++i) b.place[(size_t)at[(size_t)i]] = (int)pos[(size_t)i];
+      for (int64_t i = 0; i < n; ++i) {
+        b.lane_q[(size_t)by_work[(size_t)i]] = b.q[(size_t)i];
+        b.place[(size_t)by_work[(size_t)i]] = (int)pos[(size_t)i];
+      }
     }
+    std::vector<int2> sorted((size_t)n);
+    for (int64_t i = 0; i < n; ++i) sorted[(size_t)pos[(size_t)i]] = b.q[(size_t)i];
+    b.q.swap(sorted);
   }
   for (VQ& v : P->vqs) v.idx = remap[v.bin][(size_t)v.idx];
 }
@@ -1033,9 +1040,10 @@ static void plan_upload(cintx_plan* P) {
   };
   size_t o_rec = take(npp * 64);
   size_t o_poff = take(npair * 4), o_pnp = take(npair * 4), o_geo = take(npair * 64);
-  std::vector<size_t> o_q(P->bins.size()), o_place(P->bins.size());
+  std::vector<size_t> o_q(P->bins.size()), o_lane(P->bins.size()), o_place(P->bins.size());
   for (size_t i = 0; i < P->bins.size(); ++i) {
     o_q[i] = take(P->bins[i].q.size() * sizeof(int2));
+    o_lane[i] = take(P->bins[i].lane_q.size() * sizeof(int2));
     o_place[i] = take(P->bins[i].place.size() * sizeof(int));
   }
   size_t o_cnt = take(P->bins.size() * 2 * 8 + 8);
@@ -1105,7 +1113,9 @@ static void plan_upload(cintx_plan* P) {
     Bin& b = P->bins[i];
     put(o_q[i], b.q.data(), b.q.size() * sizeof(int2));
     b.d_q = (int2*)(P->blob + o_q[i]);
+    put(o_lane[i], b.lane_q.data(), b.lane_q.size() * sizeof(int2));
     put(o_place[i], b.place.data(), b.place.size() * sizeof(int));
+    b.d_lane_q = b.place.empty() ? nullptr : (int2*)(P->blob + o_lane[i]);
     b.d_place = b.place.empty() ? nullptr : (int*)(P->blob + o_place[i]);
   }
   HIPCHK(hipMemcpyAsync(P->blob, h.data(), host_bytes, hipMemcpyHostToDevice, C.stream));
@@ -1301,10 +1311,11 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   const KernelInfo& k = jk ? variant_info_jk(P, b, b.variant) : variant_info(P, b, b.variant);
   const PairDev pd{P->d_rec, P->d_poff, P->d_pnp, P->d_geo};
   double* scratch = b.runtime_class() ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
-  launch_bin_kernels(P->family, b.l, b.variant, b.runtime_class(), k, pd, P->expcutoff, b.d_q,
-                     b.d_place, (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(),
-                     b.most, scratch,
-                     count ? P->d_counters + 2 * i : nullptr, st, jk);
+  const bool lanes = b.d_place && !b.runtime_class() && k.lanes_per_tuple == 1;
+  launch_bin_kernels(P->family, b.l, b.variant, b.runtime_class(), k, pd, P->expcutoff,
+                     lanes ? b.d_lane_q : b.d_q, lanes ? b.d_place : nullptr,
+                     (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), b.most,
+                     scratch, count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
 
 // Spinor families: the Cartesian blocks (all bins done) -> `out`.
@@ -2980,8 +2991,8 @@ static void jk_enqueue(cintx_plan* plan, const double* Dsym, double* dJ, double*
       continue;
     }
     plan_launch_bin(plan, i, plan->d_out, false, st, chain);
-    HIPCHK(launch_jk_digest(plan->d_out, b.out_base, b.block, b.d_q, b.d_place,
-                            (int64_t)b.q.size(), plan->d_pair_sh, plan->d_ao_off, plan->d_shl_l, Dsym, dJ, dK, nao,
+    HIPCHK(launch_jk_digest(plan->d_out, b.out_base, b.block, b.d_q, (int64_t)b.q.size(),
+                            plan->d_pair_sh, plan->d_ao_off, plan->d_shl_l, Dsym, dJ, dK, nao,
                             st));
   }
   if (ev) {

@@ -994,3 +994,43 @@ def test_small_launches_of_the_runtime_class_kernel(oracle, count):
     check_plan(oracle, "int2e_sph", tuples, mol)
     check_plan(oracle, "int2e_ip1_sph", tuples[:40], mol)
     check_plan(oracle, "int2e_cart", tuples[:40], mol)
+
+
+def test_wide_shapes_list_tuples_by_primitive_counts():
+    """nabla_i (p p|p p) tuples of 36 surviving primitive tuples each, 36 x 1
+    and 1 x 36 of them in turn.  A wide shape loops to the largest counts of
+    its workgroup's tuples, so a workgroup of both kinds runs 1296 steps
+    instead of 36: the mixed list has to take about as long as both halves
+    (three times as long at most)."""
+    mol = M.Molecule()
+    at = [mol.add_atom(1, r) for r in ((0, 0, 0), (0.3, 0.2, 0), (0, 0.4, 0.1), (0.2, 0, 0.3))]
+    for a in at:
+        for e in ([0.3, 0.4, 0.5, 0.7, 0.9, 1.2], [0.6]):
+            mol.add_shell(a, 1, e, [[M.gto_norm(1, v) for v in e]])
+    mol.build()
+    long, short = [0, 2, 4, 6], [1, 3, 5, 7]
+    rng = np.random.default_rng(7)
+    halves = [[(*(int(v) for v in rng.choice(b, 2)), *(int(v) for v in rng.choice(k, 2)))
+               for _ in range(8000)] for b, k in ((long, short), (short, long))]
+
+    def best(tuples, v):
+        p = capi.Plan("int2e_ip1_sph", mol.atm, mol.bas, mol.env, tuples)
+        p.set_variant(v)
+        lanes = p.bin_variants()[0]["lanes"]
+        ms = []
+        for _ in range(6):
+            assert capi.lib().cintx_plan_execute_timed(p.h, None) == 0
+            ms.append(p.bin_stats()[0]["ms"])
+        p.close()
+        return lanes, min(ms)
+
+    seen = 0
+    for v in range(capi.NVARIANTS):
+        lanes, mixed = best([t for pair in zip(*halves) for t in pair], v)
+        if lanes == 1:
+            continue
+        seen += 1
+        parts = [best(h, v)[1] for h in halves]
+        say(f"  {lanes} lanes: {mixed:.3f} ms, halves {parts[0]:.3f} + {parts[1]:.3f}")
+        assert mixed <= 3 * sum(parts)
+    assert seen >= 2
