@@ -284,6 +284,34 @@ static void build_spinor_table(const std::vector<double>& c2s, std::vector<doubl
 // ------------------------------------------------------------------
 constexpr int kChains = 8;  // parallel chains of a captured plan graph
 
+// The launch shapes that cintx_plan_autotune found for a class, by the
+// binary logarithm of the surviving primitive tuples of the bin it timed; -1:
+// none.  A shape that wins on a long list loses on a short one ((d d|d p),
+// 56,000 primitive tuples: runtime-class kernel 0.31 ms, the wide shape that
+// wins on millions 0.43 ms), so only bins of about the same size (a factor
+// of two to four) start from it.  Plans of several threads read and write it.
+struct TunedShapes {
+  static constexpr int kSizes = 40;
+  std::atomic<signed char> shape[kSizes];
+  TunedShapes() {
+    for (auto& v : shape) v.store(-1, std::memory_order_relaxed);
+  }
+  static int size(int64_t total) {
+    return total < 1 ? 0 : std::min(63 - __builtin_clzll((unsigned long long)total), kSizes - 1);
+  }
+  int find(int64_t total) const {
+    const int n = size(total);
+    for (int k : {n, n - 1, n + 1}) {
+      const int v = k < 0 || k >= kSizes ? -1 : shape[k].load(std::memory_order_relaxed);
+      if (v >= 0) return v;
+    }
+    return -1;
+  }
+  void record(int64_t total, int v) {
+    shape[size(total)].store((signed char)v, std::memory_order_relaxed);
+  }
+};
+
 struct DevCtx {
   int device = -1;
   hipStream_t stream = nullptr;
@@ -296,8 +324,8 @@ struct DevCtx {
   Registry* reg = nullptr;
   double* d_jk_scratch = nullptr;  // the static scratch of cintx_plan_jk_noalloc
   hipEvent_t jk_ev[kChains] = {};  // fork/join events of cintx_plan_jk_noalloc's chains
-  // autotuned class-kernel variant per (deriv, form, class); -1: untuned
-  signed char tuned[2][kForms][kMaxL + 1][kMaxL + 1][kMaxL + 1][kMaxL + 1];
+  // autotuned launch shapes per (deriv, form, class)
+  TunedShapes tuned[2][kForms][kMaxL + 1][kMaxL + 1][kMaxL + 1][kMaxL + 1];
 };
 
 static std::atomic<DevCtx*> g_ctx{nullptr};
@@ -343,7 +371,6 @@ static DevCtx& ctx() {
   c->reg = new Registry();
   std::memset(c->reg, 0, sizeof(Registry));
   register_class_kernels(*c->reg);
-  std::memset(c->tuned, -1, sizeof c->tuned);
   g_ctx.store(c, std::memory_order_release);
   return *c;
 }
@@ -561,7 +588,8 @@ struct Bin {
   double prim_tuples = 0;       // from the last work count
   double flops = 0;
   bool generic = false;  // no compile-time instantiation: runtime-class kernel
-  bool small = false;    // may run the runtime-class kernel, its default
+  bool small = false;    // may run the runtime-class kernel, its default by the size rule
+  int64_t total = 0;     // surviving primitive tuples
   int64_t most = 0;      // primitive tuples of its longest tuple (runtime-class launches)
   bool runtime_class() const;  // the launch shape in use is the runtime-class kernel
   int variant = 0;       // class-kernel variant (launch shape) in use
@@ -862,6 +890,7 @@ static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_
 static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);
 static const KernelInfo& variant_info(const cintx_plan* P, const Bin& b, int v);
 static int bin_form(const cintx_plan* P, const Bin& b);
+static TunedShapes& tuned_shapes(const cintx_plan* P, const Bin& b);
 
 // A bin's blocks are placed, and its tuples listed, by (bra, ket)
 // primitive-pair counts (counting sort), or for the classes of
@@ -906,16 +935,14 @@ static void plan_sort_bins(cintx_plan* P) {
         key[(size_t)i] = std::min(S.np[b.q[i].x], 64) * 65 + std::min(S.np[b.q[i].y], 64);
       counting_sort(key, pos);
     }
-    if (!placed_by_work && !one_lane && !b.generic && b.variant < 0) {
-      int64_t total = 0, most = 0;
+    int64_t total = 0, most = 0;
+    if (!placed_by_work && !one_lane && !b.generic)
       for (const int2& v : b.q) {
         const int64_t w = surviving_prims(S, v.x, v.y, b.l[0] + b.l[1] + f.deriv, b.l[2] + b.l[3],
                                           f.three, P->expcutoff);
         total += w;
         most = std::max(most, w);
       }
-      b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
-    }
     if (placed_by_work || one_lane) {
       // by survivors alone, so that within equal survivor counts the
       // enumeration's bra-major order stays and neighbouring lanes often
@@ -929,15 +956,18 @@ static void plan_sort_bins(cintx_plan* P) {
             surviving_prims(S, b.q[i].x, b.q[i].y, lij, lkl, f.three, P->expcutoff),
             kSurvCap - 1);
       const std::vector<int64_t> first = counting_sort(key, placed_by_work ? pos : by_work);
-      const int64_t most = (int64_t)first.size() - 2;
-      int64_t total = 0;
+      most = (int64_t)first.size() - 2;
       for (int64_t w = 1; w <= most; ++w) total += w * (first[(size_t)w + 1] - first[(size_t)w]);
       split_lanes(n, total, [&](int64_t w) { return first[(size_t)std::min(w, most + 1)]; },
                   b.lanes_end.data());
-      if (b.variant < 0) b.variant = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
     }
-    b.variant = std::max(b.variant, 0);
-    b.small = b.variant == kRuntimeClass;
+    if (!b.generic) {
+      const int rule = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
+      const int v = tuned_shapes(P, b).find(total);
+      b.total = total;
+      b.small = rule == kRuntimeClass;
+      b.variant = (v == kRuntimeClass ? b.small : variant_info(P, b, v).fn != nullptr) ? v : rule;
+    }
     if (!by_work.empty()) {
       if (n > INT32_MAX) fail(CINTX_STATUS_MEMORY_LIMIT_EXCEEDED, "too many tuples of one class");
       b.lane_q.resize((size_t)n);
@@ -1176,7 +1206,7 @@ static const KernelInfo& variant_info_jk(const cintx_plan* P, const Bin& b, int 
   return ctx().reg->jk[0][b.l[0]][b.l[1]][b.l[2]][b.l[3]][v - kVariants];
 }
 
-static signed char& tuned_slot(const cintx_plan* P, const Bin& b) {
+static TunedShapes& tuned_shapes(const cintx_plan* P, const Bin& b) {
   const FamilyInfo& f = kFam[P->family];
   return ctx().tuned[f.deriv][bin_form(P, b)][b.l[0]][b.l[1]][b.l[2]][b.l[3]];
 }
@@ -1190,10 +1220,7 @@ static void plan_drop_graph(cintx_plan* P) {
 
 static void plan_check_kernels(cintx_plan* P) {
   for (auto& b : P->bins) {
-    const KernelInfo* ks = bin_kernels(P, b);
-    b.generic = (ks[0].fn == nullptr);
-    const int v = tuned_slot(P, b);
-    b.variant = (v >= 0 && variant_info(P, b, v).fn) ? v : -1;  // -1: plan_sort_bins chooses
+    b.generic = bin_kernels(P, b)[0].fn == nullptr;
   }
 }
 
@@ -1682,9 +1709,9 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   split_lanes(nq, total, [&](int64_t w) { return most < w ? nq : 0; }, lanes_end);
   int variant = 0;
   if (!generic) {
-    const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]];
-    variant = (v >= 0 && v < kVariants && ks[v].fn) ? v
-                                                    : default_variant(ks, cl, f.deriv, nq, total, most);
+    const int rule = default_variant(ks, cl, f.deriv, nq, total, most);
+    const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]].find(total);
+    variant = (v == kRuntimeClass ? rule == v : v >= 0 && v < kVariants && ks[v].fn) ? v : rule;
     if (variant == kRuntimeClass) {
       generic = true;
       variant = 0;
@@ -2569,8 +2596,7 @@ int cintx_plan_autotune(cintx_plan* plan, int reps) {
       }
       b.variant = best;
       b.last_ms = best_ms;
-      // (the runtime-class kernel wins by the size of this bin: no record)
-      if (best != kRuntimeClass) tuned_slot(plan, b) = (signed char)best;
+      tuned_shapes(plan, b).record(b.total, best);
     }
   });
 }

@@ -262,8 +262,9 @@ int cintx_plan_work(cintx_plan *plan, double *prim_tuples, double *root_evals, d
  * Every class has up to six compiled variants (lanes per tuple, primitive
  * tuples per step); cintx_plan_autotune times each on the plan's own bin
  * (min of `reps` launches after one warm-up, HIP events), keeps the fastest
- * per bin and records it for the process, so later plans of the same class
- * start from it.  Results of all variants agree to rounding (summation order
+ * per bin and records it for the process, so later plans start from it in
+ * bins of the same class and about the same number of surviving primitive
+ * tuples.  Results of all variants agree to rounding (summation order
  * of the primitive loop differs).  The FP32 bins of a mixed plan also try the
  * FP64 instantiations (variants 6..11 = FP64 variant 0..5): FP32 without packed
  * math issues at the FP64 rate on CDNA4 and wins only where it saves

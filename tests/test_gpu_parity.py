@@ -898,6 +898,36 @@ def test_autotune_keeps_results(oracle):
     p.close()
 
 
+def test_autotuned_shapes_stay_with_their_size():
+    """Autotuning a long list of a class leaves the launch shapes of a short
+    list of long tuples of that class as they are."""
+    mol = M.Molecule()
+    for r in ((0, 0, 0), (1.1, 0.2, 0), (0.1, 1.3, 0.4)):
+        a = mol.add_atom(1, r)
+        for e in ([3.0, 0.9, 0.3], [1.4, 0.5]):
+            mol.add_shell(a, 2, e, [[M.gto_norm(2, v) for v in e]])
+    mol.build()
+    rng = np.random.default_rng(3)
+
+    def plan(shells, count):
+        return capi.Plan("int2e_sph", mol.atm, mol.bas, mol.env,
+                         [tuple(int(s) for s in rng.choice(shells, 4)) for _ in range(count)])
+
+    def shapes():  # 3 tuples of 81 primitive tuples
+        p = plan([0, 2, 4], 3)
+        got = [(b["generic"], v["variant"], v["lanes"], v["prims"])
+               for b, v in zip(p.bin_stats(), p.bin_variants())]
+        p.close()
+        return got
+
+    before = shapes()
+    p = plan([1, 3, 5], 6000)  # of 16 each
+    p.autotune(reps=1)
+    say(f"  short list {before}, long list {p.bin_variants()}")
+    p.close()
+    assert shapes() == before
+
+
 @pytest.mark.parametrize("variant", range(capi.NVARIANTS))
 def test_work_counters_match_oracle_model(oracle, variant):
     """The device work counters (surviving primitive tuples after libcint's
