@@ -608,6 +608,10 @@ int64_t generic_scratch(const int* l, int deriv, int64_t nq, int64_t most) {
   return S.per * (S.split ? nq : std::min<int64_t>(nq, kGenericGrid));
 }
 
+int generic_prims_per_step(const int* l, int deriv, int64_t nq, int64_t most) {
+  return gen_split(l, deriv, nq, most).P;
+}
+
 hipError_t launch_generic(const EriArgs& a, const int* l, int deriv, int64_t most,
                           hipStream_t s) {
   const GenShape S = gen_split(l, deriv, a.nq, most);

@@ -34,6 +34,7 @@ hipError_t launch_rys_eval(const RysTable& tab, int n, const double* x, int64_t 
 hipError_t launch_generic(const EriArgs& a, const int* l, int deriv, int64_t most,
                           hipStream_t s);
 int64_t generic_scratch(const int* l, int deriv, int64_t nq, int64_t most);
+int generic_prims_per_step(const int* l, int deriv, int64_t nq, int64_t most);
 hipError_t mlp_train_device(const RysTable& tab, float* prm, int64_t nsamples, int epochs,
                             int batch, float lr, uint64_t seed, double* final_loss,
                             hipStream_t st);
@@ -2628,7 +2629,10 @@ int cintx_plan_bin_variants(const cintx_plan* plan, int64_t nmax, int* variant, 
       if (variant) variant[i] = b.generic ? -1 : rc ? nv : b.variant;
       if (nvariants) nvariants[i] = nv + (b.small ? 1 : 0);
       if (lanes) lanes[i] = rc ? 256 : k.lanes_per_tuple;
-      if (prims) prims[i] = rc ? 1 : k.prims_per_step;
+      if (prims)
+        prims[i] = rc ? generic_prims_per_step(b.l, kFam[plan->family].deriv,
+                                               (int64_t)b.q.size(), b.most)
+                      : k.prims_per_step;
       if (tuples_per_block) tuples_per_block[i] = rc ? 1 : k.tuples_per_block;
     }
   });

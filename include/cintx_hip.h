@@ -270,11 +270,17 @@ int cintx_plan_work(cintx_plan *plan, double *prim_tuples, double *root_evals, d
  * math issues at the FP64 rate on CDNA4 and wins only where it saves
  * registers or LDS bytes.  cintx_plan_set_variant forces one variant (0..5)
  * on every bin that has it (variant 0 otherwise).  Untuned bins choose by
- * their size; a small bin may take the runtime-class kernel, which then is
- * one more variant of that bin, the last.  cintx_plan_bin_variants reports per
- * bin: variant in use (-1: a class that has only the runtime-class kernel),
- * variants available, lanes per tuple, primitive tuples per step (for one lane per
- * tuple: row chunks), tuples per workgroup. */
+ * their size; a small bin may take the runtime-class kernel, which is then
+ * one more variant of that bin: reported with the number after the last
+ * compiled one, tried by the autotuner, not selected by
+ * cintx_plan_set_variant.  cintx_plan_bin_variants reports per bin: variant
+ * in use (-1: a class that has only the runtime-class kernel), variants
+ * available, lanes per tuple, primitive tuples per step (for one lane per
+ * tuple: row chunks), tuples per workgroup.  For the runtime-class kernel
+ * the lanes are those of a workgroup, of which several may share a tuple of
+ * a short list; a one-lane kernel spreads a long tuple over up to 64 lanes.
+ * A bin of the FP32 precision runs in FP64 where its variant is one of
+ * 6..11 or the runtime-class kernel. */
 int cintx_plan_autotune(cintx_plan *plan, int reps);
 int cintx_plan_set_variant(cintx_plan *plan, int variant);
 int cintx_plan_bin_variants(const cintx_plan *plan, int64_t nmax, int *variant, int *nvariants,

@@ -898,6 +898,29 @@ def test_autotune_keeps_results(oracle):
     p.close()
 
 
+def _two_site_shells(l, nprim, r):
+    """One shell of momentum l with nprim primitives on each of two sites."""
+    mol = M.Molecule()
+    for x in (0.0, r):
+        a = mol.add_atom(1, (x, 0.1 * x, 0.0))
+        e = [0.7 * 1.2 ** k for k in range(nprim)]
+        mol.add_shell(a, l, e, [[M.gto_norm(l, v) for v in e]])
+    return mol.build()
+
+
+def test_bin_variants_report_the_runtime_class_kernel():
+    """The primitive tuples of a step of the runtime-class kernel: several
+    where the tuples have several and their g tensors fit, never more than
+    the tuples have."""
+    for nprim, want in ((1, (1, 1)), (2, (2, 16)), (4, (2, 16))):
+        mol = _two_site_shells(3, nprim, 1.0)
+        p = capi.Plan("int2e_ip1_sph", mol.atm, mol.bas, mol.env, [(0, 1, 0, 1), (1, 0, 1, 1)])
+        for b, v in zip(p.bin_stats(), p.bin_variants()):
+            assert b["generic"] and v["variant"] == -1 and v["lanes"] == 256
+            assert want[0] <= v["prims"] <= want[1], (nprim, v)
+        p.close()
+
+
 def test_autotuned_shapes_stay_with_their_size():
     """Autotuning a long list of a class leaves the launch shapes of a short
     list of long tuples of that class as they are."""
