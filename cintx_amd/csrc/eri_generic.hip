@@ -29,6 +29,7 @@ struct GenShape {
   int level;   // rows per lane (gen_rows_per_lane)
   bool glds;
   int lds;     // doubles of dynamic LDS
+  int slabs;   // slabs that a workgroup finishes at a time (not split)
   int64_t per;  // scratch doubles per workgroup, or per tuple when split
 };
 
@@ -211,13 +212,17 @@ __device__ __forceinline__ void gout_rows(const double* gp, const int* ox, const
   }
 }
 
-// The finish of a block, slab by slab (the elements of one Cartesian component
-// fl of shell l): a slab always fits in LDS, and slabs can go to different
+// The finish of a block, by slabs (the elements of one Cartesian component fl
+// of shell l): a slab always fits in LDS, and slabs can go to different
 // workgroups.  part: [nslice][ncomp][nf] partial blocks.
 //
-// generic_slab: the sum of the slices' slabs, the i, j and k axes turned into
-// spherical harmonics in `lds` (two slabs), left in the slab's place in slice
-// 0.  generic_last: the elements [e0, e1) of one component of the spherical
+// generic_slabs: for the nfl slabs from fl on, the sum of the slices' slabs,
+// the i, j and k axes turned into spherical harmonics in `lds` (twice nfl
+// slabs), left in the slabs' places in slice 0.  A workgroup that finishes a
+// whole block takes as many at a time as its LDS holds: each pass is a chain
+// of global reads, up to four barriers and writes (5,000 nabla_i (s s|g g)
+// tuples of one primitive tuple, 15 slabs each: 0.89 ms one by one, 0.27 ms
+// all at once).  generic_last: the elements [e0, e1) of one component of the spherical
 // block: the l axis, as a weighted sum over the slabs, and the strided write.
 __device__ __forceinline__ double* generic_out(const EriArgs& a, int64_t q, int comp) {
   return a.out + a.out_base + q * a.block + comp * a.st_comp;
@@ -227,20 +232,20 @@ __device__ __forceinline__ int generic_slab_size(const GenShape& S) {
   return ncart(S.l[0]) * ncart(S.l[1]) * ncart(S.l[2]);
 }
 
-__device__ void generic_slab(const EriArgs& a, const GenShape& S, double* part, int comp, int fl,
-                             double* lds) {
+__device__ void generic_slabs(const EriArgs& a, const GenShape& S, double* part, int comp, int fl,
+                              int nfl, double* lds) {
   const int t = threadIdx.x, T = blockDim.x;
   const int n = generic_slab_size(S);
   double* at = part + (size_t)comp * S.nf + (size_t)fl * n;
-  for (int e = t; e < n; e += T) {
+  for (int e = t; e < nfl * n; e += T) {
     double v = at[e];
     for (int s = 1; s < S.nslice; ++s) v += at[(size_t)s * S.ncomp * S.nf + e];
     lds[e] = v;
   }
   __syncthreads();
-  int dims[4] = {ncart(S.l[0]), ncart(S.l[1]), ncart(S.l[2]), 1};
+  int dims[4] = {ncart(S.l[0]), ncart(S.l[1]), ncart(S.l[2]), nfl};
   double* src = lds;
-  double* dst = lds + n;
+  double* dst = lds + nfl * n;
   for (int ax = 0; ax < 3; ++ax) {
     if (S.l[ax] < 2 || a.cart) continue;
     c2s_pass_mfma(dst, src, dims, ax, S.l[ax], a.c2s, t, T);
@@ -251,7 +256,7 @@ __device__ void generic_slab(const EriArgs& a, const GenShape& S, double* part, 
     __syncthreads();
   }
   const int ns = dims[0] * dims[1] * dims[2];
-  for (int e = t; e < ns; e += T) at[e] = src[e];
+  for (int e = t; e < nfl * ns; e += T) at[(e / ns) * n + e % ns] = src[e];
   __syncthreads();
 }
 
@@ -295,7 +300,7 @@ __global__ void __launch_bounds__(256) eri_generic_slab_kernel(EriArgs a, GenSha
   const int64_t b = blockIdx.x / nfl;
   const int fl = (int)(blockIdx.x - b * nfl);
   const int64_t q = b / S.ncomp;
-  generic_slab(a, S, a.scratch + (size_t)q * S.per, (int)(b - q * S.ncomp), fl, gl);
+  generic_slabs(a, S, a.scratch + (size_t)q * S.per, (int)(b - q * S.ncomp), fl, 1, gl);
 }
 __global__ void __launch_bounds__(256) eri_generic_last_kernel(EriArgs a, GenShape S, int pieces) {
   const int64_t b = blockIdx.x / pieces;
@@ -536,7 +541,8 @@ __global__ void __launch_bounds__(256, gen_waves(DERIV, LEVEL))
     }
     if (!S.split) {
       for (int comp = 0; comp < S.ncomp; ++comp) {
-        for (int fl = 0; fl < nfl; ++fl) generic_slab(a, S, part, comp, fl, gl);
+        for (int fl = 0; fl < nfl; fl += S.slabs)
+          generic_slabs(a, S, part, comp, fl, min(S.slabs, nfl - fl), gl);
         generic_last(a, S, q, part, comp, 0, generic_out_size(a, S));
       }
       __syncthreads();
@@ -594,8 +600,14 @@ static GenShape gen_split(const int* l, int deriv, int64_t nq, int64_t most) {
     S.split = S.nslice * S.nchunk > 1 && bytes() <= ((int64_t)256 << 20);
     if (!S.split) S.nslice = 1;
   }
-  S.lds = std::max((S.glds ? S.P * gsz : 0) + S.P * per_prim,
-                   S.split ? 0 : 2 * ncart(l[0]) * ncart(l[1]) * ncart(l[2]));
+  S.lds = (S.glds ? S.P * gsz : 0) + S.P * per_prim;
+  S.slabs = 1;
+  if (!S.split) {  // room for more slabs, short of what costs a workgroup per CU
+    const int slab = 2 * ncart(l[0]) * ncart(l[1]) * ncart(l[2]);
+    const int free_lds = gen_waves(deriv != 0, S.level) == 2 ? two / 2 : cap;
+    S.lds = std::max({S.lds, slab, std::min(ncart(l[3]) * slab, free_lds)});
+    S.slabs = std::min(ncart(l[3]), S.lds / slab);
+  }
   S.per = (int64_t)S.nslice * S.ncomp * S.nf +
           (S.glds ? 0 : (S.split ? (int64_t)S.nslice * S.nchunk : 1) * gsz);
   S.per = (S.per + 31) / 32 * 32;

@@ -921,6 +921,37 @@ def test_bin_variants_report_the_runtime_class_kernel():
         p.close()
 
 
+def test_runtime_class_blocks_finish_several_slabs_at_a_time(oracle):
+    """Blocks finished by the workgroup that made them, with one slab, with
+    all slabs in one pass and with a remainder; and nabla_i (s s|g g), 15
+    slabs, in about the time of (g g|s s), one slab of as many elements (it
+    took 3.3 times as long slab by slab; 2 at most)."""
+    mol = M.Molecule()
+    for r in ((0, 0, 0), (0.9, 0.3, 0)):
+        a = mol.add_atom(1, r)
+        for l in range(5):
+            e = 0.5 + 0.2 * l
+            mol.add_shell(a, l, [e], [[M.gto_norm(l, e)]])
+    mol.build()
+    for ls in ((4, 4, 0, 0), (0, 0, 4, 4), (2, 4, 1, 4), (2, 4, 4, 3), (4, 3, 4, 4), (0, 4, 2, 2)):
+        t = (ls[0], ls[1] + 5, ls[2], ls[3] + 5)
+        check_plan(oracle, "int2e_ip1_sph", [t, t], mol)
+
+    def best(ls):
+        p = capi.Plan("int2e_ip1_sph", mol.atm, mol.bas, mol.env,
+                      [(ls[0], ls[1] + 5, ls[2], ls[3] + 5)] * 5000)
+        ms = []
+        for _ in range(8):
+            assert capi.lib().cintx_plan_execute_timed(p.h, None) == 0
+            ms.append(p.bin_stats()[0]["ms"])
+        p.close()
+        return min(ms)
+
+    many, one = best((0, 0, 4, 4)), best((4, 4, 0, 0))
+    say(f"  15 slabs {many:.3f} ms, one slab {one:.3f} ms")
+    assert many <= 2 * one
+
+
 def test_autotuned_shapes_stay_with_their_size():
     """Autotuning a long list of a class leaves the launch shapes of a short
     list of long tuples of that class as they are."""
