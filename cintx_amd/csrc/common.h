@@ -91,6 +91,7 @@ struct EriArgs {
   int64_t block;           // elements per block (components included)
   int64_t nq;
   LaneSplit split;         // one-lane kernels
+  bool few_prims;          // their launch: too few primitive tuples per lane for a table in LDS
   double common;           // pi^3 2/sqrt(pi) prod common_fac_sp
   double expcutoff;
   int lij_ceil, lkl_ceil;  // li_ceil+lj_ceil, lk_ceil+ll_ceil for the screen

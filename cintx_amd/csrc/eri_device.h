@@ -464,6 +464,11 @@ struct ClassShape {
   // libcint's fixed base loses up to 1e-10 in FP64)
   static constexpr bool PB = (PP >> 13) & 1;
   static_assert(!PB || (TT > 1 && !JK), "per-primitive transfer base: wide path, no J/K");
+  // one-lane kernels of up to 3 roots copy the table block of their n (14 to
+  // 53 KB) to LDS once per workgroup: the coefficient reads of every root
+  // then hit LDS instead of scattered L2 lines.  PP bit 14: not where a lane
+  // has too few primitive tuples for that (launch_class)
+  static constexpr bool TABLE_IN_LDS = TT == 1 && NR <= 3 && !((PP >> 14) & 1);
   static constexpr int nout(int l) { return CART ? ncart(l) : nsph(l); }
   static constexpr int RPC = (NROW + NCH - 1) / NCH;  // rows per chunk
   static constexpr int G = T >= NROW ? T / NROW : 1;               // groups per row
@@ -599,10 +604,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   (void)lds;
   constexpr bool F64 = sizeof(R) == sizeof(double);
   constexpr int NCH = S::NCH, RPC = S::RPC, CE = RPC * NB;  // elements per chunk
-  // up to 3 roots the table block of this n (<= 53 KB) is copied to LDS once
-  // per workgroup: the coefficient reads of every root then hit LDS instead
-  // of scattered L2 lines
-  constexpr bool LTAB = NR <= 3;
+  constexpr bool LTAB = S::TABLE_IN_LDS;
   __shared__ __attribute__((aligned(16))) double stab[LTAB ? rys_block_doubles(NR) : 2];
   const double* coefn = a.rys.coef + a.rys.off[NR];
   if constexpr (LTAB) {
@@ -1305,6 +1307,13 @@ hipError_t launch_class(const EriArgs& a, hipStream_t s) {
     static_assert(S::jk_lds_bytes() + (S::NR <= 3 ? rys_block_doubles(S::NR) * 8 : 0) <= 160 * 1024,
                   "fused J/K staging");
     dyn = S::jk_lds_bytes();
+  }
+  if constexpr (S::TABLE_IN_LDS && !S::JK) {
+    if (a.few_prims) {
+      hipLaunchKernelGGL((eri_class_kernel<LI, LJ, LK, LL, DERIV, R, TT, PP | 16384>),
+                         dim3((unsigned)nblk), dim3(S::T * Q), dyn, s, a);
+      return hipGetLastError();
+    }
   }
   hipLaunchKernelGGL((eri_class_kernel<LI, LJ, LK, LL, DERIV, R, TT, PP>), dim3((unsigned)nblk),
                      dim3(S::T * Q), dyn, s, a);

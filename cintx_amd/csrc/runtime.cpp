@@ -1237,7 +1237,7 @@ struct PairDev {
 // slots) and form prec, blocks of `block` elements written from out_base.
 // Variant `k` of the compiled class kernels, or the runtime-class kernel
 // (generic, tuples of at most `most` primitive tuples) with `scratch` of
-// generic_scratch doubles.
+// generic_scratch doubles.  `total`: surviving primitive tuples.
 // Fused J/K of a launch: the class kernel digests its blocks into J/K.
 struct JkFuse {
   const double* D;
@@ -1252,7 +1252,7 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
                                const KernelInfo& k, const PairDev& pd, double expcutoff,
                                const int2* d_q, const int* d_place, int64_t nq, double* out,
                                int64_t out_base, int64_t block, const int64_t* lanes_end,
-                               int64_t most, double* scratch,
+                               int64_t total, int64_t most, double* scratch,
                                unsigned long long* counters, hipStream_t st,
                                const JkFuse* jk = nullptr) {
   DevCtx& C = ctx();
@@ -1293,6 +1293,15 @@ static void launch_bin_kernels(int fam, const int* l, int variant, bool generic,
     a.ao_off = jk->ao_off;
     a.nao = jk->nao;
   }
+  // Copying the Rys table to LDS takes a workgroup as long as about two
+  // primitive tuples a lane: with one or less (uncontracted shells) the
+  // one-lane kernels read it where it is.  int2c2e_sph (s|g), 24,576 pairs,
+  // 0.0135 ms with the copy and 0.0113 ms without; with two to four primitive
+  // tuples a lane both take the same, with eight the copy wins by 5%.
+  int64_t nlane = 0;
+  for (int r = 0; r < kSplits; ++r)
+    nlane += (std::min(nq, lanes_end[r]) - (r > 0 ? std::min(nq, lanes_end[r - 1]) : 0)) << r;
+  a.few_prims = total <= nlane;
   // a dispatch holds at most 2^32 - 1 work-items per grid dimension: launch
   // in chunks of at most 2^31 lanes (all tuples for the runtime-class
   // kernel, whose grid is capped anyway; 2^24 for the one-lane kernels, of
@@ -1342,8 +1351,8 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   const bool lanes = b.d_place && !b.runtime_class() && k.lanes_per_tuple == 1;
   launch_bin_kernels(P->family, b.l, b.variant, b.runtime_class(), k, pd, P->expcutoff,
                      lanes ? b.d_lane_q : b.d_q, lanes ? b.d_place : nullptr,
-                     (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), b.most,
-                     scratch, count ? P->d_counters + 2 * i : nullptr, st, jk);
+                     (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), b.total,
+                     b.most, scratch, count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
 
 // Spinor families: the Cartesian blocks (all bins done) -> `out`.
@@ -1760,7 +1769,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   double* dout = (double*)(A + o_out);
   unsigned long long* dcnt = (unsigned long long*)(A + o_cnt);
   launch_bin_kernels(fam, cl, variant, generic, ks[variant], pd, cutoff,
-                     (const int2*)(A + o_q), nullptr, nq, dout, 0, block, lanes_end, longest,
+                     (const int2*)(A + o_q), nullptr, nq, dout, 0, block, lanes_end, total, longest,
                      generic ? (double*)(A + o_scr) : nullptr, dcnt, T.stream);
   int d[4] = {n[0], n[1], n[2], n[3]};
   if (dims)

@@ -1045,6 +1045,35 @@ def test_lanes_shared_by_a_tuple(oracle, count):
         p.close()
 
 
+@pytest.mark.parametrize("count", [1, 255, 257])
+def test_one_primitive_tuple_per_lane(oracle, count):
+    """Lists of uncontracted shells, whose one-lane kernels read the Rys table
+    from memory: every output form, 1 to 3 roots and more, arguments from 0
+    to beyond the table, a last workgroup of one lane; and beside contracted
+    shells on the other side of the rule."""
+    mol = M.Molecule()
+    rng = np.random.default_rng(60 + count)
+    for r in ((0, 0, 0), (0.7, 0.2, 0.1), (0.3, 9.0, 2.0)):
+        a = mol.add_atom(1, r)
+        for l in range(3):
+            for e in (0.3, 1.7, 900.0):
+                mol.add_shell(a, l, [e], [[M.gto_norm(l, e)]])
+    contracted = mol.add_atom(1, (1.0, 0.4, 0.3))
+    for l in range(2):
+        e = [20.0, 4.0, 1.0, 0.4]
+        mol.add_shell(contracted, l, e, [[M.gto_norm(l, v) for v in e]])
+    mol.build()
+    n = 27
+    one = [s for s in range(n) if mol.bas[s, 1] < 2]
+    t4 = [tuple(int(v) for v in rng.choice(one, 4)) for _ in range(count)]
+    t3 = [tuple(int(v) for v in rng.integers(0, n, 3)) for _ in range(count)]
+    t2 = [t[:2] for t in t3]
+    for name, t in (("int2e_sph", t4), ("int2e_cart", t4), ("int2e_ip1_sph", t4),
+                    ("int3c2e_sph", t3), ("int3c2e_ip1_sph", t3), ("int2c2e_sph", t2),
+                    ("int2e_sph", t4 + [(n, n + 1, n, n)] * 40)):
+        check_plan(oracle, name, t, mol)
+
+
 @pytest.mark.parametrize("count", [1, 7, 300])
 def test_small_launches_of_the_runtime_class_kernel(oracle, count):
     """Classes with compiled kernels whose small launches take the
