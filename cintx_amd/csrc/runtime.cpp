@@ -855,7 +855,11 @@ inline bool Bin::runtime_class() const { return generic || variant == kRuntimeCl
 // primitive tuples, 0.038 ms against 0.061 ms in the wide kernel; (d p|d),
 // 233,000, 0.067 against 0.084; (d d|p), 87,000, 0.053 against 0.040; (d p|f),
 // 175,000 in two chunks, 0.17 against 0.10; (d p|p) nabla_i, 13,000 in two,
-// 0.07 against 0.03.
+// 0.07 against 0.03.  There is no line for classes of at most 51 registers or
+// of a single row, whose wide kernels have one lane with elements: int3c2e_sph
+// (d d|s), 125 to 1,134 tuples, 0.025 ms against 0.044 to 0.073; (p s|d), 67
+// to 1,481 tuples, 0.018 against 0.034 to 0.048.  (Uncontracted tuples of
+// several rows keep it: int2c2e_sph (p|d), 3,060 pairs, 0.011 against 0.008.)
 //
 // Long tuples are what the wide kernels, which walk a tuple a few primitive
 // tuples at a time, are worst at; the one-lane kernels spread one over up to
@@ -885,7 +889,8 @@ static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_
                       (deriv ? 3 : 1) / nch;
   const int64_t size = (g + acc) * nch;
   if (is_long) return size >= 125 && splits && total < 75 * size ? kRuntimeClass : one;
-  return other < 0 || total >= 700 * size ? one : other;
+  const int rows = ncart(l[2]) * ncart(l[3]) * (deriv ? ncart(l[1]) : 1);
+  return other < 0 || rows == 1 || (size <= 51 && most > 1) || total >= 700 * size ? one : other;
 }
 
 static const KernelInfo* bin_kernels(const cintx_plan* P, const Bin& b);

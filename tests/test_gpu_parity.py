@@ -952,6 +952,29 @@ def test_runtime_class_blocks_finish_several_slabs_at_a_time(oracle):
     assert many <= 2 * one
 
 
+def test_default_shape_of_short_lists(oracle):
+    """Short lists of short contracted tuples of classes whose wide kernels
+    would keep one lane busy, or of few registers, run the one-lane kernel;
+    uncontracted pairs of several rows the wide one."""
+    mol = M.Molecule()
+    rng = np.random.default_rng(17)
+    for r in ((0, 0, 0), (1.0, 0.3, 0.2)):
+        a = mol.add_atom(1, r)
+        for l in range(3):
+            e = [4.0, 1.1, 0.4]
+            mol.add_shell(a, l, e, [[rng.normal() * M.gto_norm(l, v) for v in e]])
+            mol.add_shell(a, l, [0.7], [[M.gto_norm(l, 0.7)]])
+    mol.build()
+    s, p, d, p1, d1 = 0, 2, 4, 3, 5  # contracted s, p, d; uncontracted p, d
+    for name, t, one in (("int3c2e_sph", (d, d + 6, s), True),
+                         ("int3c2e_sph", (p, s + 6, d), True),
+                         ("int2c2e_sph", (p1, d1), False)):
+        plan = capi.Plan(name, mol.atm, mol.bas, mol.env, [t] * 100)
+        assert (plan.bin_variants()[0]["lanes"] == 1) == one, (name, t)
+        plan.close()
+        check_plan(oracle, name, [t] * 3, mol)
+
+
 def test_autotuned_shapes_stay_with_their_size():
     """Autotuning a long list of a class leaves the launch shapes of a short
     list of long tuples of that class as they are."""
