@@ -243,9 +243,13 @@ def variants(deriv, prec, ls):
         # components (or nabla_i) the most lanes with several primitive
         # tuples in flight.  They lose at most 5% to fewer lanes on large
         # launches and win up to 3 times on small ones ((d d|p p), 8,462
-        # tuples: 0.57 ms with 64 lanes, 2.04 ms with 16).
+        # tuples: 0.57 ms with 64 lanes, 2.04 ms with 16).  Not where more
+        # lanes mean fewer primitive tuples in flight than the first shape
+        # has: (d p|p s), 18 to 31,085 tuples, takes 1.2 to 1.6 times as long
+        # with 32 lanes and 3 as with 16 and 5.
         rows = [c for c in out if c[1] & 256] if nrow < 16 else []
-        many = sorted((c for c in out if c[0] > 1 and 1 < c[1] < 256), key=lambda c: -c[0])
+        many = sorted((c for c in out if c[0] > 1 and max(2, pw) <= c[1] < 256),
+                      key=lambda c: -c[0])
         for c in (rows or many)[:1]:
             out.remove(c)
             out.insert(0, c)

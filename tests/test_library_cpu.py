@@ -153,6 +153,16 @@ def test_gto_norm_reference_known_answer():
     assert abs(M.gto_norm(0, 0.5) - 1.502251088929885) < 1e-12
 
 
+@pytest.mark.parametrize("deriv,ls", [(0, (2, 1, 1, 0)), (0, (2, 2, 0, 0)),
+                                      (1, (2, 0, 1, 0)), (1, (2, 1, 0, 0))])
+def test_default_wide_shape_keeps_primitive_tuples_in_flight(deriv, ls):
+    """The default wide shape of classes with few rows is not one of more
+    lanes and fewer primitive tuples per step."""
+    from cintx_amd import build as B
+    wide = [(tt, pp & 255) for tt, pp in B.variants(deriv, 0, ls) if tt > 1]
+    assert wide[0][0] == 16 and wide[0][1] >= 5, wide
+
+
 def test_build_variant_rules():
     """The launch-shape rules of the f/g templates (cintx_amd/build.py):
     classes within the LDS-staging and chain-register limits, kets pairing an
