@@ -86,7 +86,7 @@ struct EriArgs {
   const double* pair_geo;  // 8 per pair: ri[3], rj[3], log(|Rij|+1), unused
   // work list
   const int2* quartets;    // (bra pair, ket pair)
-  const int* place;        // one-lane kernels: block of every tuple (null: its own number)
+  const int* place;        // block of every tuple (null: its own number; wide kernels always)
   int64_t out_base;        // element offset of this launch's first block
   int64_t block;           // elements per block (components included)
   int64_t nq;

@@ -225,7 +225,7 @@ __device__ __forceinline__ void gout_rows(const double* gp, const int* ox, const
 // all at once).  generic_last: the elements [e0, e1) of one component of the spherical
 // block: the l axis, as a weighted sum over the slabs, and the strided write.
 __device__ __forceinline__ double* generic_out(const EriArgs& a, int64_t q, int comp) {
-  return a.out + a.out_base + q * a.block + comp * a.st_comp;
+  return a.out + a.out_base + (a.place ? a.place[q] : q) * a.block + comp * a.st_comp;
 }
 
 __device__ __forceinline__ int generic_slab_size(const GenShape& S) {

@@ -597,9 +597,9 @@ struct Bin {
   std::vector<int2> q;
   int64_t out_base = 0;  // element offset of the bin's first block
   int64_t block = 0;     // elements per block (NS * ncomp)
-  // one-lane launches: their order of the tuples and the block of each, where
-  // that is not the order of q, and the tuples before lanes_end[k], which take
-  // at most 2^k lanes
+  // the tuples in the order of their surviving primitive tuples and the block
+  // of each, where that is not the order of q, and for one-lane launches the
+  // tuples before lanes_end[k], which take at most 2^k lanes
   std::vector<int2> lane_q;
   std::vector<int> place;
   std::array<int64_t, kSplits> lanes_end{};
@@ -901,10 +901,11 @@ static TunedShapes& tuned_shapes(const cintx_plan* P, const Bin& b);
 // A bin's blocks are placed, and its tuples listed, by (bra, ket)
 // primitive-pair counts (counting sort), or for the classes of
 // Registry::by_work by surviving primitive tuples (stable).  A class with a
-// one-lane kernel that is not one of those has a second list for it, by
-// surviving primitive tuples: the lanes of a wavefront, which each walk their
-// own survivors, then run equal numbers of iterations and neighbouring tuples
-// take equal numbers of lanes.  (The wide kernels' workgroups loop to the
+// one-lane kernel that is not one of those has a second list, by surviving
+// primitive tuples, for it and for the runtime-class kernel: the lanes of a
+// wavefront, which each walk their own survivors, then run equal numbers of
+// iterations and neighbouring tuples take equal numbers of lanes, and the
+// runtime-class kernel starts its longest tuples first.  (The wide kernels' workgroups loop to the
 // largest counts among their tuples, and on that list, where equal numbers of
 // survivors come of different counts, nabla_i (p p|p p) of 4 to 541 tuples
 // took up to 1.5 times as long as on the other.)
@@ -1353,9 +1354,9 @@ static void plan_launch_bin(cintx_plan* P, size_t i, double* out, bool count,
   const KernelInfo& k = jk ? variant_info_jk(P, b, b.variant) : variant_info(P, b, b.variant);
   const PairDev pd{P->d_rec, P->d_poff, P->d_pnp, P->d_geo};
   double* scratch = b.runtime_class() ? P->d_scratch + (size_t)chain * (size_t)P->scratch_stride : nullptr;
-  const bool lanes = b.d_place && !b.runtime_class() && k.lanes_per_tuple == 1;
+  const bool by_work = b.d_place && (b.runtime_class() || k.lanes_per_tuple == 1);
   launch_bin_kernels(P->family, b.l, b.variant, b.runtime_class(), k, pd, P->expcutoff,
-                     lanes ? b.d_lane_q : b.d_q, lanes ? b.d_place : nullptr,
+                     by_work ? b.d_lane_q : b.d_q, by_work ? b.d_place : nullptr,
                      (int64_t)b.q.size(), out, b.out_base, b.block, b.lanes_end.data(), b.total,
                      b.most, scratch, count ? P->d_counters + 2 * i : nullptr, st, jk);
 }
