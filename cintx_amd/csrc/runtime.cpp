@@ -872,9 +872,15 @@ inline bool Bin::runtime_class() const { return generic || variant == kRuntimeCl
 // equal.  It keeps more of the chip busy for it, so beside the other bins of a
 // plan it pays at a quarter of those sizes: int2e_ip1_sph, 300,000 tuples of
 // 18 atoms, 4.3 ms with the lines below and 5.8 ms with four times as large
-// ones; the integrals of 3 atoms 0.8 ms, and 2.9 ms without it.
+// ones; the integrals of 3 atoms 0.8 ms, and 2.9 ms without it.  A launch
+// alone (`alone`: a plan of one class, a single call) has the lines at half
+// of that, where the two kernels' own times cross over all classes of five
+// molecules: nabla_i (s d|d d), 256 tuples, 12,800 in all, 0.49 ms against
+// 0.29 ms wide; (d p|d p), 602 tuples, 12,200, 0.29 against 0.14.  (In plans
+// of many classes, halved lines cost the integrals of 3 atoms 29% and
+// int2e_ip2_sph of 18 atoms, 50,000 tuples, 15%.)
 static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_t nq,
-                           int64_t total, int64_t most) {
+                           int64_t total, int64_t most, bool alone) {
   int one = -1, other = -1;
   for (int v = kVariants - 1; v >= 0; --v) {
     if (!ks[v].fn) continue;
@@ -882,13 +888,15 @@ static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_
   }
   const bool is_long = most >= 64;
   const bool splits = nq < kGenFew;  // the runtime-class kernel's tuples go to several workgroups
-  if (one < 0) return is_long && splits && total < 20000 ? kRuntimeClass : std::max(other, 0);
+  const int half = alone ? 2 : 1;
+  if (one < 0)
+    return is_long && splits && total < 20000 / half ? kRuntimeClass : std::max(other, 0);
   const int64_t nch = ks[one].prims_per_step;
   const int64_t g = 3LL * (l[0] + deriv + 1) * (l[1] + 1) * (l[2] + 1) * (l[3] + 1);
   const int64_t acc = (int64_t)ncart(l[0]) * ncart(l[1]) * ncart(l[2]) * ncart(l[3]) *
                       (deriv ? 3 : 1) / nch;
   const int64_t size = (g + acc) * nch;
-  if (is_long) return size >= 125 && splits && total < 75 * size ? kRuntimeClass : one;
+  if (is_long) return size >= 125 && splits && total < 75 * size / half ? kRuntimeClass : one;
   const int rows = ncart(l[2]) * ncart(l[3]) * (deriv ? ncart(l[1]) : 1);
   return other < 0 || rows == 1 || (size <= 51 && most > 1) || total >= 700 * size ? one : other;
 }
@@ -969,7 +977,8 @@ static void plan_sort_bins(cintx_plan* P) {
                   b.lanes_end.data());
     }
     if (!b.generic) {
-      const int rule = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most);
+      const int rule = default_variant(bin_kernels(P, b), b.l, f.deriv, n, total, most,
+                                       P->bins.size() == 1);
       const int v = tuned_shapes(P, b).find(total);
       b.total = total;
       b.small = rule == kRuntimeClass;
@@ -1725,7 +1734,7 @@ static int raw_eval(int fam, double* out, const int* dims, const int* shls, cons
   split_lanes(nq, total, [&](int64_t w) { return most < w ? nq : 0; }, lanes_end);
   int variant = 0;
   if (!generic) {
-    const int rule = default_variant(ks, cl, f.deriv, nq, total, most);
+    const int rule = default_variant(ks, cl, f.deriv, nq, total, most, true);
     const int v = C.tuned[f.deriv][f.cart ? 2 : 0][cl[0]][cl[1]][cl[2]][cl[3]].find(total);
     variant = (v == kRuntimeClass ? rule == v : v >= 0 && v < kVariants && ks[v].fn) ? v : rule;
     if (variant == kRuntimeClass) {

@@ -975,6 +975,26 @@ def test_default_shape_of_short_lists(oracle):
         check_plan(oracle, name, [t] * 3, mol)
 
 
+def test_list_of_one_class_has_the_lines_of_a_launch_alone(oracle):
+    """240 nabla_i (s d|d d) tuples of 54 to 81 primitive tuples, 13,000 to
+    19,440 in all: the compiled kernel when the list has no other class, the
+    runtime-class kernel beside another."""
+    mol = M.Molecule()
+    for r in ((0, 0, 0), (0.8, 0.3, 0.2)):
+        a = mol.add_atom(1, r)
+        for l in (0, 2):
+            e = [2.0, 0.9, 0.4]
+            mol.add_shell(a, l, e, [[M.gto_norm(l, v) for v in e]])
+    mol.build()
+    t = [(0, 1, 3, 1), (2, 3, 1, 3), (0, 3, 1, 1)] * 80
+    for tuples, generic in ((t, False), (t + [(0, 0, 0, 2)], True)):
+        p = capi.Plan("int2e_ip1_sph", mol.atm, mol.bas, mol.env, tuples)
+        got = {b["class"]: b["generic"] for b in p.bin_stats()}
+        p.close()
+        assert got[(0, 2, 2, 2)] == generic, got
+    check_plan(oracle, "int2e_ip1_sph", t, mol)
+
+
 def test_autotuned_shapes_stay_with_their_size():
     """Autotuning a long list of a class leaves the launch shapes of a short
     list of long tuples of that class as they are."""
