@@ -898,6 +898,32 @@ def test_autotune_keeps_results(oracle):
     p.close()
 
 
+def test_mixed_jk_with_runtime_class_bins(oracle):
+    """J/K of a mixed plan whose bins digest in fused kernels and from blocks
+    of the runtime-class kernel, against the CPU J/K of the same quartets."""
+    rng = M.SplitMix64(5)
+    mol = M.Molecule()
+    atoms = [mol.add_atom(8, r) for r in M._lattice(rng, 2, 2, 2, 2.8, 0.3)]
+    M._orbital_basis(mol, rng, atoms, [True] * len(atoms), 0.1, 5000.0)
+    mol.build()
+    p = capi.Plan("int2e_sph", mol.atm, mol.bas, mol.env, screened=(1e-12, 4),
+                  precision=capi.PREC_MIXED, mixed_threshold=1e-9)
+    kinds = {(b["precision"], b["generic"]) for b in p.bin_stats()}
+    say(f"  {p.ntuples} quartets, {p.ntuples_fp32} in FP32, bins {sorted(kinds)}")
+    assert p.ntuples_fp32 > 0 and {True, False} == {g for _, g in kinds}
+    nao = mol.nao()
+    D = np.random.default_rng(8).normal(size=(nao, nao)) / nao
+    D = D + D.T
+    t, _ = p.tuples()
+    Jc, Kc = oracle.cpu_baseline_jk(t, mol.atm, mol.bas, mol.env, D, nthreads=16)
+    for _ in range(2):
+        J, K = p.jk(D)
+        ej, ek = float(np.abs(J - Jc).max()), float(np.abs(K - Kc).max())
+        say(f"  J/K vs CPU: {ej:.3e} {ek:.3e} (|J| {np.abs(Jc).max():.3e})")
+        assert ej <= 1e-10 and ek <= 1e-10
+    p.close()
+
+
 def _two_site_shells(l, nprim, r):
     """One shell of momentum l with nprim primitives on each of two sites."""
     mol = M.Molecule()
