@@ -75,9 +75,9 @@ def high_l_classes():
     most HIGH_L_MAX_NF Cartesian elements and HIGH_L_MAX_G4 values per
     recurrence chain, FP64 only, without Cartesian or
     fused-J/K copies.  Their blocks are small, so the runtime-class kernel
-    (one tuple per 256-lane workgroup, one primitive tuple per step) leaves
-    most of its lanes idle on them; the template kernels batch tuples and
-    primitive tuples instead.  A bra whose f or g shell pairs with a shell
+    (a 256-lane workgroup works on one tuple, up to 16 primitive tuples per
+    step) leaves many of its lanes idle on long lists of them; the template
+    kernels batch tuples as well.  A bra whose f or g shell pairs with a shell
     of l >= 2 runs the wide path with the transfer base chosen per
     primitive tuple (needs_pb); libcint's fixed base loses up to 1e-10 in
     FP64 there (144x the 1e-12 bar on (g g|s s) tuples of the s..g

@@ -50,7 +50,7 @@ __host__ __device__ constexpr void cart_decode(int l, int c, int& lx, int& ly, i
 // place: one step of third order from v_rsq_f64 (23 bits), with the rounding
 // of v y carried along.  A division and a square root, with their scaling
 // and fix-up steps, take three times the instructions, which counts where
-// the vector units bound a kernel: they are 58 to 75% busy in the one-lane
+// the vector units bound a kernel: they are 55 to 79% busy in the one-lane
 // kernels, and (p s|p s), 1,733,629 tuples, 1.10e8 primitive tuples, took
 // 1.41 ms with both and the Chebyshev sums, 1.23 ms with the table alone
 // changed and takes 1.07 ms.
@@ -578,8 +578,9 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
   unsigned int nsurv = 0;
 
   // Primitive counts are per tuple; a workgroup of several tuples loops to
-  // its largest counts (tuples are sorted by (npij, npkl) so that is rarely
-  // more) and masks the excess iterations.
+  // its largest counts and masks the excess iterations.  (Tuples are listed
+  // by (npij, npkl), so that is rarely more, or for small classes by surviving
+  // primitive tuples: plan_sort_bins.)
   const int np_ij = a.pair_np[pq.x], np_kl = a.pair_np[pq.y];
   int mij = np_ij, mkl = np_kl;
   if constexpr (T > 1) {
@@ -730,7 +731,7 @@ __global__ void __launch_bounds__((ClassShape<LI, LJ, LK, LL, DERIV, TT, PP>::T 
 #pragma unroll
         for (int kk = 0; kk < ACC; ++kk) part[kk] = 0;
       }
-      // small blocks: all roots first (their Clenshaw recurrences interleave),
+      // small blocks: all roots first (their Horner sums interleave),
       // then one root at a time through the chains and the elements; larger
       // blocks evaluate each root in turn to keep registers for g
       constexpr bool ROOTS_FIRST = 3 * G4 * (int)sizeof(R) / 8 + ACC <= 64;

@@ -2818,8 +2818,9 @@ int cintx_plan_create_screened(cintx_plan** plan, const int* atm, int natm, cons
           qof[((uint64_t)s.a << 32) | (uint32_t)s.b] = {
               qabs[(size_t)s.id], transfer_growth(atm, bas, env, s.a, s.b)};
         // FP32 without packed math issues at the FP64 rate on CDNA4: the FP32
-        // recurrences pay only in classes that must share g through LDS (half
-        // the LDS bytes and registers), which are those not placed by work
+        // recurrences pay only in classes that share g through LDS (half the
+        // LDS bytes and registers).  Those are the classes not placed by work;
+        // of them (d d|d s) and a few more have a chunked one-lane kernel too
         auto fp32_pays = [&](const int* sh) {
           int la = B.l[sh[0]], lb = B.l[sh[1]], lc = B.l[sh[2]], ld = B.l[sh[3]];
           if (lc > la || (lc == la && ld > lb)) {
