@@ -869,7 +869,11 @@ inline bool Bin::runtime_class() const { return generic || variant == kRuntimeCl
 // where a launch is small and the one-lane kernel large or missing: (d p|p p),
 // 150 tuples, 30,000 in all, 0.12 ms against 0.19 ms one-lane; (d d|d p), 400
 // tuples, 56,000, 0.31 ms against 0.43 ms wide; (d p|d p), 820 tuples, 80,000,
-// equal.  It keeps more of the chip busy for it, so beside the other bins of a
+// equal.  A one-lane kernel of three row chunks, which evaluates every root
+// three times, leaves long tuples to the wide kernel below 400 primitive
+// tuples per register: nabla_i (p d|d s), 1,194 tuples, 53,000 in all, 0.51
+// ms against 0.25 ms; (d d|p s), 177,000, 0.38 against 0.32, and 270,000, 0.45
+// against 0.54.  The runtime-class kernel keeps more of the chip busy for it, so beside the other bins of a
 // plan it pays at a quarter of those sizes: int2e_ip1_sph, 300,000 tuples of
 // 18 atoms, 4.3 ms with the lines below and 5.8 ms with four times as large
 // ones; the integrals of 3 atoms 0.8 ms, and 2.9 ms without it.  A launch
@@ -896,7 +900,8 @@ static int default_variant(const KernelInfo* ks, const int* l, int deriv, int64_
   const int64_t acc = (int64_t)ncart(l[0]) * ncart(l[1]) * ncart(l[2]) * ncart(l[3]) *
                       (deriv ? 3 : 1) / nch;
   const int64_t size = (g + acc) * nch;
-  if (is_long) return size >= 125 && splits && total < 75 * size / half ? kRuntimeClass : one;
+  if (is_long && size >= 125 && splits && total < 75 * size / half) return kRuntimeClass;
+  if (is_long) return nch == 3 && other >= 0 && total < 400 * size ? other : one;
   const int rows = ncart(l[2]) * ncart(l[3]) * (deriv ? ncart(l[1]) : 1);
   return other < 0 || rows == 1 || (size <= 51 && most > 1) || total >= 700 * size ? one : other;
 }

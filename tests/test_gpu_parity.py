@@ -1021,6 +1021,27 @@ def test_list_of_one_class_has_the_lines_of_a_launch_alone(oracle):
     check_plan(oracle, "int2e_ip1_sph", t, mol)
 
 
+def test_three_row_chunks_leave_long_tuples_to_the_wide_kernel(oracle):
+    """nabla_i (p d|d s), whose one-lane kernel works in three row chunks:
+    1,200 tuples of 54 or 81 primitive tuples run the wide kernel, (p p|d s),
+    of two chunks, the one-lane kernel."""
+    mol = M.Molecule()
+    for r in ((0, 0, 0), (0.8, 0.3, 0.2)):
+        a = mol.add_atom(1, r)
+        for l in range(3):
+            e = [2.0, 0.9, 0.4]
+            mol.add_shell(a, l, e, [[M.gto_norm(l, v) for v in e]])
+    mol.build()
+    s, p, d = 0, 1, 2
+    for j, one in ((d, False), (p, True)):
+        t = [(p, j + 3, d, s), (p + 3, j, d, s + 3), (p, j, d + 3, s)] * 400
+        plan = capi.Plan("int2e_ip1_sph", mol.atm, mol.bas, mol.env, t)
+        assert plan.nbins == 1 and not plan.bin_stats()[0]["generic"]
+        assert (plan.bin_variants()[0]["lanes"] == 1) == one, j
+        plan.close()
+        check_plan(oracle, "int2e_ip1_sph", t[:60], mol)
+
+
 def test_autotuned_shapes_stay_with_their_size():
     """Autotuning a long list of a class leaves the launch shapes of a short
     list of long tuples of that class as they are."""
