@@ -873,10 +873,11 @@ inline bool Bin::runtime_class() const { return generic || variant == kRuntimeCl
 // three times, leaves long tuples to the wide kernel below 400 primitive
 // tuples per register: nabla_i (p d|d s), 1,194 tuples, 53,000 in all, 0.51
 // ms against 0.25 ms; (d d|p s), 177,000, 0.38 against 0.32, and 270,000, 0.45
-// against 0.54.  The runtime-class kernel keeps more of the chip busy for it, so beside the other bins of a
-// plan it pays at a quarter of those sizes: int2e_ip1_sph, 300,000 tuples of
-// 18 atoms, 4.3 ms with the lines below and 5.8 ms with four times as large
-// ones; the integrals of 3 atoms 0.8 ms, and 2.9 ms without it.  A launch
+// against 0.54.  The runtime-class kernel keeps more of the chip busy for its
+// time, so beside the other bins of a plan it pays at a quarter of those
+// sizes: int2e_ip1_sph, 300,000 tuples of 18 atoms, 4.3 ms with the lines
+// below and 5.8 ms with four times as large ones; the integrals of 3 atoms
+// 0.8 ms, and 2.9 ms without it.  A launch
 // alone (`alone`: a plan of one class, a single call) has the lines at half
 // of that, where the two kernels' own times cross over all classes of five
 // molecules: nabla_i (s d|d d), 256 tuples, 12,800 in all, 0.49 ms against
@@ -918,10 +919,10 @@ static TunedShapes& tuned_shapes(const cintx_plan* P, const Bin& b);
 // primitive tuples, for it and for the runtime-class kernel: the lanes of a
 // wavefront, which each walk their own survivors, then run equal numbers of
 // iterations and neighbouring tuples take equal numbers of lanes, and the
-// runtime-class kernel starts its longest tuples first.  (The wide kernels' workgroups loop to the
-// largest counts among their tuples, and on that list, where equal numbers of
-// survivors come of different counts, nabla_i (p p|p p) of 4 to 541 tuples
-// took up to 1.5 times as long as on the other.)
+// runtime-class kernel starts its longest tuples first.  (The wide kernels'
+// workgroups loop to the largest counts among their tuples, and on that list,
+// where equal numbers of survivors come of different counts, nabla_i (p p|p p)
+// of 4 to 541 tuples took up to 1.5 times as long as on the other.)
 static void plan_sort_bins(cintx_plan* P) {
   const PairSet& S = P->pairs;
   const FamilyInfo& f = kFam[P->family];
